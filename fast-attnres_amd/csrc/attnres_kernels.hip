@@ -72,6 +72,15 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// the same 16 and 8 bytes at element (2-byte), FP32 or byte alignment
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
+typedef f32x4 f32x4_at4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_at2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_at1 __attribute__((aligned(1)));
+typedef uint32_t u32_at2 __attribute__((aligned(2)));
+typedef uint32_t u32_at1 __attribute__((aligned(1)));
+typedef uint16_t u16_at1 __attribute__((aligned(1)));
 
 // ------------------------------------------------------------- BF16 helpers
 
@@ -95,15 +104,91 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float acc) {
 template <int G>
 __device__ __forceinline__ int chunk_start(int c, int lane) { return (c * G + lane) * kVec; }
 
+// First element a lane actually touches for the chunk that starts at d0.
+// Aligned rows (VEC) hold whole chunks.  Other rows -- a base, stride or width
+// that is no multiple of 16 bytes -- take the same 16-byte accesses at element
+// alignment (the hardware runs with unaligned access enabled), and a row whose
+// width is no multiple of 8 ends in a chunk moved back to the row's last 8
+// elements: it repeats 8 - D % 8 elements of the chunk before it, which the
+// sums mask out (own_mask) and the stores leave to that chunk.  So no lane
+// touches a byte outside its row.  Measured on MI355X: a copy with loads and
+// stores 2 bytes off alignment moves 5.4 TB/s against 6.2 aligned.  One
+// element per access, as these rows were read before, took (forward /
+// backward us, before -> now): S = 13, N = 4095, D = 1537, R = 385: 121 -> 48 /
+// 222 -> 83; S = 25, N = 4096, D = 2048, rows 2049 apart: 230 -> 86 / 447 ->
+// 166; S = 9, N = 4096, D = 4095: 201 -> 77 / 1500 -> 163 (the element-wise
+// 4096-wide backward spilled); S = 12, N = 8192, D = 300, rows 301 apart: 49
+// -> 28 / 79 -> 50.
+// Rows of fewer than 8 elements (the 16-lane geometry) go element by element.
+template <bool VEC>
+__device__ __forceinline__ int chunk_pos(int d0, int D) {
+  if constexpr (VEC) {
+    return d0;
+  } else {
+    return max(min(d0, D - kVec), 0);
+  }
+}
+
+// Row element at position i of a row laid out by chunks (chunk i / 8, element
+// i % 8), or a value past the row where that chunk does not hold it.
+template <bool VEC>
+__device__ __forceinline__ int element_at(int i, int D) {
+  if constexpr (VEC) {
+    return i;
+  } else {
+    const int d0 = i & ~(kVec - 1);
+    const int d = chunk_pos<VEC>(d0, D) + (i & (kVec - 1));
+    return d >= d0 ? d : D;
+  }
+}
+
+// Row element of the first half of word j of a lane's chunk c.
+template <int G, bool VEC>
+__device__ __forceinline__ int word_pos(int c, int lane, int j, int D) {
+  if constexpr (VEC) {
+    return chunk_start<G>(c, lane) + 2 * j;
+  } else {
+    return chunk_pos<VEC>(chunk_start<G>(c, lane), D) + 2 * j;
+  }
+}
+
+// All ones on the halves of that word (row elements d, d + 1) that belong to
+// the chunk itself and not, in an unaligned row, to the chunk before it.
+template <int G, bool VEC>
+__device__ __forceinline__ uint32_t own_mask(int c, int lane, int d) {
+  if constexpr (VEC) {
+    return 0xffffffffu;
+  } else {
+    const int d0 = chunk_start<G>(c, lane);
+    return (d >= d0 ? 0x0000ffffu : 0u) | (d + 1 >= d0 ? 0xffff0000u : 0u);
+  }
+}
+
 // Load one row (this lane's chunks) as raw packed BF16 words.  Every load is
 // unconditional: a chunk that starts at or beyond D reads the row's first
-// chunk instead, and callers neutralise such lanes with the word masks of
-// key_masks / range_masks (branch-free loads keep several rows in flight;
-// a conditional load would join control flow and force a wait for it).
-// VEC requires 16-byte aligned rows and D % 8 == 0 (so D >= 8).
+// chunk (VEC) or its last 8 elements instead, and callers neutralise such
+// lanes with the word masks of key_masks / range_masks (branch-free loads keep
+// several rows in flight; a conditional load would join control flow and force
+// a wait for it).  VEC requires 16-byte aligned rows and D % 8 == 0 (so D >= 8).
 template <int G, int CH, bool VEC>
 __device__ __forceinline__ void load_row(const uint16_t* __restrict__ row, int lane, int D,
                                          u32x4 (&raw)[CH]) {
+  if constexpr (!VEC && G == 16) {
+    if (D < kVec) {  // uniform
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t lo = row[min(2 * j, D - 1)];
+          const uint32_t hi = row[min(2 * j + 1, D - 1)];
+          w[j] = lo | (hi << 16);
+        }
+        raw[c] = u32x4{w[0], w[1], w[2], w[3]};
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     const int d0 = chunk_start<G>(c, lane);
@@ -111,15 +196,7 @@ __device__ __forceinline__ void load_row(const uint16_t* __restrict__ row, int l
       const int at = d0 < D ? d0 : 0;
       raw[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + at));
     } else {
-      uint32_t w[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int d = d0 + 2 * j;
-        const uint32_t lo = row[d < D ? d : D - 1];
-        const uint32_t hi = row[d + 1 < D ? d + 1 : D - 1];
-        w[j] = lo | (hi << 16);
-      }
-      raw[c] = u32x4{w[0], w[1], w[2], w[3]};
+      raw[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_at2*>(row + chunk_pos<VEC>(d0, D)));
     }
   }
 }
@@ -138,6 +215,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t row_resource(const void* row, 
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(row), static_cast<short>(0), bytes, 0x00020000);
 }
 
+//
+// Store the chunk that starts at d0 < D.  An unaligned row's last chunk, which
+// repeats elements of the chunk before it (chunk_pos), stores its own D % 8
+// elements only, as 8, 4 and 2 bytes from the row's end.
 template <int G, bool VEC>
 __device__ __forceinline__ void store_chunk(uint16_t* __restrict__ row, int d0, int D, const u32x4& w) {
   if constexpr (VEC && G >= 64) {
@@ -145,11 +226,58 @@ __device__ __forceinline__ void store_chunk(uint16_t* __restrict__ row, int d0, 
   } else if constexpr (VEC) {
     __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(row + d0));
   } else {
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+    if constexpr (G == 16) {
+      if (D < kVec) {  // uniform
+        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-    for (int e = 0; e < kVec; ++e) {
-      if (d0 + e < D) {
-        row[d0 + e] = static_cast<uint16_t>((e & 1) ? (ws[e >> 1] >> 16) : (ws[e >> 1] & 0xffffu));
+        for (int e = 0; e < kVec; ++e) {
+          if (d0 + e < D) {
+            row[d0 + e] = static_cast<uint16_t>((e & 1) ? (ws[e >> 1] >> 16) : (ws[e >> 1] & 0xffffu));
+          }
+        }
+        return;
+      }
+    }
+    if (d0 + kVec <= D) {
+      __builtin_nontemporal_store(w, reinterpret_cast<u32x4_at2*>(row + d0));
+    } else {
+      const int own = D & (kVec - 1);  // uniform
+      if (own & 4) *reinterpret_cast<u32x2_at2*>(row + D - 4) = u32x2{w.z, w.w};
+      if (own & 2) *reinterpret_cast<u32_at2*>(row + D - (own & 4) - 2) = (own & 4) ? w.y : w.w;
+      if (own & 1) {
+        const uint32_t pair = (own & 4) ? ((own & 2) ? w.x : w.y) : ((own & 2) ? w.z : w.w);
+        row[D - own] = static_cast<uint16_t>(pair >> 16);
+      }
+    }
+  }
+}
+
+// The same for the chunk's 8 refinement bytes.
+template <int G, bool VEC>
+__device__ __forceinline__ void store_refine(int8_t* __restrict__ refine, int d0, int D, const u32x2& r) {
+  if constexpr (VEC && G >= 64) {
+    __builtin_amdgcn_raw_buffer_store_b64(r, row_resource(refine, D), d0, 0, kStoreScNt);
+  } else if constexpr (VEC) {
+    __builtin_nontemporal_store(r, reinterpret_cast<u32x2*>(refine + d0));
+  } else {
+    if constexpr (G == 16) {
+      if (D < kVec) {  // uniform
+#pragma unroll
+        for (int e = 0; e < kVec; ++e) {
+          if (d0 + e < D) refine[d0 + e] = static_cast<int8_t>(((e < 4 ? r.x : r.y) >> (8 * (e & 3))) & 0xffu);
+        }
+        return;
+      }
+    }
+    if (d0 + kVec <= D) {
+      __builtin_nontemporal_store(r, reinterpret_cast<u32x2_at1*>(refine + d0));
+    } else {
+      const int own = D & (kVec - 1);  // uniform
+      if (own & 4) *reinterpret_cast<u32_at1*>(refine + D - 4) = r.y;
+      if (own & 2) *reinterpret_cast<u16_at1*>(refine + D - (own & 4) - 2) = static_cast<uint16_t>(((own & 4) ? r.x : r.y) >> 16);
+      if (own & 1) {  // byte 8 - own of the chunk: the odd byte of its pair
+        const uint32_t word = (own & 4) ? r.x : r.y;
+        refine[D - own] = static_cast<int8_t>((own & 2) ? (word >> 8) : (word >> 24));
       }
     }
   }
@@ -194,17 +322,7 @@ __device__ __forceinline__ void store_row_refined(uint16_t* __restrict__ row, in
       }
     }
     store_chunk<G, VEC>(row, d0, D, u32x4{w[0], w[1], w[2], w[3]});
-    if constexpr (!REFINE) {
-    } else if constexpr (VEC && G >= 64) {
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{r[0], r[1]}, row_resource(refine, D), d0, 0, kStoreScNt);
-    } else if constexpr (VEC) {
-      __builtin_nontemporal_store(u32x2{r[0], r[1]}, reinterpret_cast<u32x2*>(refine + d0));
-    } else {
-#pragma unroll
-      for (int e = 0; e < kVec; ++e) {
-        if (d0 + e < D) refine[d0 + e] = static_cast<int8_t>((r[e >> 2] >> (8 * (e & 3))) & 0xffu);
-      }
-    }
+    if constexpr (REFINE) store_refine<G, VEC>(refine, d0, D, u32x2{r[0], r[1]});
     __builtin_amdgcn_sched_barrier(0);  // encode one chunk at a time (register pressure)
   }
 }
@@ -213,7 +331,7 @@ __device__ __forceinline__ void store_row_refined(uint16_t* __restrict__ row, in
 // key coordinates, +0 elsewhere (including d >= D).  The loads are
 // unconditional (clamped index) and masked afterwards, so none of them sits
 // behind a branch.
-template <int G, int CH>
+template <int G, int CH, bool VEC>
 __device__ __forceinline__ void load_query_words(const uint16_t* __restrict__ query, int lane, int D,
                                                  int tail0, uint32_t (&qw)[CH][4]) {
   const int R = D - tail0;
@@ -221,40 +339,42 @@ __device__ __forceinline__ void load_query_words(const uint16_t* __restrict__ qu
   for (int c = 0; c < CH; ++c) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int d = chunk_start<G>(c, lane) + 2 * j;
+      const int d = word_pos<G, VEC>(c, lane, j, D);
       const uint32_t lo = query[min(max(d - tail0, 0), R - 1)];
       const uint32_t hi = query[min(max(d + 1 - tail0, 0), R - 1)];
       const uint32_t mask = ((d >= tail0 && d < D) ? 0x0000ffffu : 0u) |
                             ((d + 1 >= tail0 && d + 1 < D) ? 0xffff0000u : 0u);
-      qw[c][j] = (lo | (hi << 16)) & mask;
+      qw[c][j] = (lo | (hi << 16)) & mask & own_mask<G, VEC>(c, lane, d);
     }
   }
 }
 
 // Word masks selecting the key coordinates (D-R <= d < D) of this lane's words.
-template <int G, int CH>
+template <int G, int CH, bool VEC>
 __device__ __forceinline__ void key_masks(int lane, int D, int tail0, uint32_t (&km)[CH][4]) {
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int d = chunk_start<G>(c, lane) + 2 * j;
-      km[c][j] = ((d >= tail0 && d < D) ? 0x0000ffffu : 0u) |
-                 ((d + 1 >= tail0 && d + 1 < D) ? 0xffff0000u : 0u);
+      const int d = word_pos<G, VEC>(c, lane, j, D);
+      km[c][j] = (((d >= tail0 && d < D) ? 0x0000ffffu : 0u) |
+                  ((d + 1 >= tail0 && d + 1 < D) ? 0xffff0000u : 0u)) &
+                 own_mask<G, VEC>(c, lane, d);
     }
   }
 }
 
-// Zero the words of this lane's chunks that lie at or beyond D.
-template <int G, int CH>
+// Zero the words of this lane's chunks that lie at or beyond D, or belong to
+// the chunk before.
+template <int G, int CH, bool VEC>
 __device__ __forceinline__ void mask_range(int lane, int D, u32x4 (&x)[CH]) {
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
-    const int d = chunk_start<G>(c, lane);
-    x[c].x &= (d < D ? 0x0000ffffu : 0u) | (d + 1 < D ? 0xffff0000u : 0u);
-    x[c].y &= (d + 2 < D ? 0x0000ffffu : 0u) | (d + 3 < D ? 0xffff0000u : 0u);
-    x[c].z &= (d + 4 < D ? 0x0000ffffu : 0u) | (d + 5 < D ? 0xffff0000u : 0u);
-    x[c].w &= (d + 6 < D ? 0x0000ffffu : 0u) | (d + 7 < D ? 0xffff0000u : 0u);
+    const int d = word_pos<G, VEC>(c, lane, 0, D);
+    x[c].x &= ((d < D ? 0x0000ffffu : 0u) | (d + 1 < D ? 0xffff0000u : 0u)) & own_mask<G, VEC>(c, lane, d);
+    x[c].y &= ((d + 2 < D ? 0x0000ffffu : 0u) | (d + 3 < D ? 0xffff0000u : 0u)) & own_mask<G, VEC>(c, lane, d + 2);
+    x[c].z &= ((d + 4 < D ? 0x0000ffffu : 0u) | (d + 5 < D ? 0xffff0000u : 0u)) & own_mask<G, VEC>(c, lane, d + 4);
+    x[c].w &= ((d + 6 < D ? 0x0000ffffu : 0u) | (d + 7 < D ? 0xffff0000u : 0u)) & own_mask<G, VEC>(c, lane, d + 6);
   }
 }
 
@@ -400,9 +520,9 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_kernel(const FwdArgs<Rows>
   if (my_tokens == 0) return;  // whole group idle (no barrier follows for it)
 
   uint32_t qw[CH][4];
-  load_query_words<G, CH>(a.query, lane, D, tail0, qw);
+  load_query_words<G, CH, VEC>(a.query, lane, D, tail0, qw);
   uint32_t km[CH][4];
-  if constexpr (!NOMASK) key_masks<G, CH>(lane, D, tail0, km);
+  if constexpr (!NOMASK) key_masks<G, CH, VEC>(lane, D, tail0, km);
 
   const int64_t last = my_tokens * S;
   const uint16_t* idle = a.src.row(0, gid);
@@ -590,9 +710,9 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_block_kernel(const FwdArgs
   }
 
   uint32_t qw[CH][4];
-  load_query_words<G, CH>(a.query, lane, D, tail0, qw);
+  load_query_words<G, CH, VEC>(a.query, lane, D, tail0, qw);
   uint32_t km[CH][4];
-  if constexpr (!NOMASK) key_masks<G, CH>(lane, D, tail0, km);
+  if constexpr (!NOMASK) key_masks<G, CH, VEC>(lane, D, tail0, km);
 
   const uint16_t* idle = a.src.row(0, tok[0]);
   u32x4 ring[NB][CH];
@@ -736,13 +856,19 @@ __device__ __forceinline__ void load_token(const BwdArgs<Rows, Grads>& a, int64_
     if constexpr (VEC) {
       t.r[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(refine + (d0 < D ? d0 : 0)));
     } else {
-      uint32_t rq[2] = {0u, 0u};
+      if constexpr (G == 16) {
+        if (D < kVec) {  // uniform
+          uint32_t rq[2] = {0u, 0u};
 #pragma unroll
-      for (int e = 0; e < kVec; ++e) {
-        const uint32_t b = static_cast<uint8_t>(refine[d0 + e < D ? d0 + e : D - 1]);
-        rq[e >> 2] |= b << (8 * (e & 3));
+          for (int e = 0; e < kVec; ++e) {
+            const uint32_t b = static_cast<uint8_t>(refine[d0 + e < D ? d0 + e : D - 1]);
+            rq[e >> 2] |= b << (8 * (e & 3));
+          }
+          t.r[c] = u32x2{rq[0], rq[1]};
+          continue;
+        }
       }
-      t.r[c] = u32x2{rq[0], rq[1]};
+      t.r[c] = __builtin_nontemporal_load(reinterpret_cast<const u32x2_at1*>(refine + chunk_pos<VEC>(d0, D)));
     }
   }
   t.run_max = a.stats[token];
@@ -791,19 +917,20 @@ __device__ __forceinline__ float token_delta(const TokenRows<CH>& t) {
 
 // The query on this workgroup's row positions, FP32, +0 off the key (every
 // group of the workgroup reads it from LDS).  Ends with a barrier.
-template <int G, int CH>
+template <int G, int CH, bool VEC>
 __device__ __forceinline__ void fill_query_lds(const uint16_t* __restrict__ query, float* q_lds, int tail0, int D,
                                                int R) {
-  for (int d = threadIdx.x; d < G * CH * kVec; d += kBlock) {
+  for (int i = threadIdx.x; i < G * CH * kVec; i += kBlock) {
+    const int d = element_at<VEC>(i, D);
     const uint32_t bits = query[min(max(d - tail0, 0), R - 1)];
-    q_lds[d] = (d >= tail0 && d < D) ? __uint_as_float(bits << 16) : 0.0f;
+    q_lds[i] = (d >= tail0 && d < D) ? __uint_as_float(bits << 16) : 0.0f;
   }
   __syncthreads();
 }
 
 // Fixed-order reduction of the groups' dq into this block's partial row
 // (`dq_lds` holds kBlock * kVec floats).  Every thread of the block calls it.
-template <int G, int CH>
+template <int G, int CH, bool VEC>
 __device__ __forceinline__ void store_dq_partial(const float (&dq)[CH][kVec], float* dq_lds, float* partial,
                                                  int group, int lane, int tail0, int D) {
   constexpr int kGroups = kBlock / G;
@@ -816,7 +943,7 @@ __device__ __forceinline__ void store_dq_partial(const float (&dq)[CH][kVec], fl
       float t = dq_lds[j];
 #pragma unroll
       for (int k = 1; k < kGroups; ++k) t += dq_lds[k * (G * kVec) + j];
-      const int d = c * G * kVec + j;
+      const int d = element_at<VEC>(c * G * kVec + j, D);
       if (d >= tail0 && d < D) partial[d - tail0] = t;
     }
     __syncthreads();
@@ -824,7 +951,7 @@ __device__ __forceinline__ void store_dq_partial(const float (&dq)[CH][kVec], fl
 }
 
 // One FP32 row (this lane's chunks, two 16-byte words each), unconditional
-// like load_row: chunks at or beyond D read the row start (VEC) or clamped
+// like load_row: chunks at or beyond D read the row start (VEC) or its last 8
 // elements.  VEC requires 16-byte aligned rows and D % 8 == 0.
 template <int G, int CH, bool VEC>
 __device__ __forceinline__ void load_row_f32(const float* __restrict__ row, int lane, int D, u32x4 (&raw)[2 * CH]) {
@@ -836,11 +963,38 @@ __device__ __forceinline__ void load_row_f32(const float* __restrict__ row, int 
       raw[2 * c] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + at));
       raw[2 * c + 1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + at + 4));
     } else {
-      uint32_t w[kVec];
+      if constexpr (G == 16) {
+        if (D < kVec) {  // uniform
+          uint32_t w[kVec];
 #pragma unroll
-      for (int e = 0; e < kVec; ++e) w[e] = __float_as_uint(row[min(d0 + e, D - 1)]);
-      raw[2 * c] = u32x4{w[0], w[1], w[2], w[3]};
-      raw[2 * c + 1] = u32x4{w[4], w[5], w[6], w[7]};
+          for (int e = 0; e < kVec; ++e) w[e] = __float_as_uint(row[min(d0 + e, D - 1)]);
+          raw[2 * c] = u32x4{w[0], w[1], w[2], w[3]};
+          raw[2 * c + 1] = u32x4{w[4], w[5], w[6], w[7]};
+          continue;
+        }
+      }
+      const u32x4_at4* at = reinterpret_cast<const u32x4_at4*>(row + chunk_pos<VEC>(d0, D));
+      raw[2 * c] = __builtin_nontemporal_load(at);
+      raw[2 * c + 1] = __builtin_nontemporal_load(at + 1);
+    }
+  }
+}
+
+// Store the 8 FP32 elements of the chunk that starts at d0 < D (an unaligned
+// row's last chunk stores its own elements only, as store_chunk does).
+template <bool VEC>
+__device__ __forceinline__ void store_chunk_f32(float* __restrict__ row, int d0, int D, const float (&x)[kVec]) {
+  if constexpr (VEC) {
+    __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<f32x4*>(row + d0));
+    __builtin_nontemporal_store(f32x4{x[4], x[5], x[6], x[7]}, reinterpret_cast<f32x4*>(row + d0 + 4));
+  } else if (d0 + kVec <= D) {
+    __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<f32x4_at4*>(row + d0));
+    __builtin_nontemporal_store(f32x4{x[4], x[5], x[6], x[7]}, reinterpret_cast<f32x4_at4*>(row + d0 + 4));
+  } else {
+    const int at = chunk_pos<VEC>(d0, D);
+#pragma unroll
+    for (int e = 0; e < kVec; ++e) {
+      if (at + e >= d0 && at + e < D) row[at + e] = x[e];
     }
   }
 }
@@ -890,9 +1044,9 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_kernel(const BwdArgs<Rows,
   const float scale = a.scale;
   int phase = 0;
 
-  fill_query_lds<G, CH>(a.query, q_lds, tail0, D, R);
+  fill_query_lds<G, CH, VEC>(a.query, q_lds, tail0, D, R);
   uint32_t km[CH][4];
-  if constexpr (!NOMASK) key_masks<G, CH>(lane, D, tail0, km);
+  if constexpr (!NOMASK) key_masks<G, CH, VEC>(lane, D, tail0, km);
   float dq[CH][kVec];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
@@ -920,7 +1074,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_kernel(const BwdArgs<Rows,
     float delta, run_max, inv_sum;
     TokenRows<CH> pend;  // rows of the next token, between request and fold
     auto fold = [&]() __attribute__((always_inline)) {
-      if constexpr (!NOMASK) mask_range<G, CH>(lane, D, pend.g);
+      if constexpr (!NOMASK) mask_range<G, CH, VEC>(lane, D, pend.g);
       float red[1] = {token_delta<CH>(pend)};
       group_sum<G, 1>(red, xred, phase);
       delta = red[0];
@@ -1049,19 +1203,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_kernel(const BwdArgs<Rows,
           }
         }
         if constexpr (kF32) {
-          if constexpr (VEC) {
-            if (NOMASK || d0 < D) {
-              __builtin_nontemporal_store(f32x4{outf[0], outf[1], outf[2], outf[3]},
-                                          reinterpret_cast<f32x4*>(grad_row + d0));
-              __builtin_nontemporal_store(f32x4{outf[4], outf[5], outf[6], outf[7]},
-                                          reinterpret_cast<f32x4*>(grad_row + d0 + 4));
-            }
-          } else {
-#pragma unroll
-            for (int e = 0; e < kVec; ++e) {
-              if (d0 + e < D) grad_row[d0 + e] = outf[e];
-            }
-          }
+          if (NOMASK || d0 < D) store_chunk_f32<VEC>(grad_row, d0, D, outf);
         } else if (NOMASK || d0 < D) {
           store_chunk<G, VEC>(grad_row, d0, D, u32x4{out[0], out[1], out[2], out[3]});
         }
@@ -1094,7 +1236,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_kernel(const BwdArgs<Rows,
     }
   }
 
-  store_dq_partial<G, CH>(dq, dq_lds, a.partial + static_cast<int64_t>(blockIdx.x) * R, group, lane, tail0, D);
+  store_dq_partial<G, CH, VEC>(dq, dq_lds, a.partial + static_cast<int64_t>(blockIdx.x) * R, group, lane, tail0, D);
 }
 
 // ---------------------------------------------------- backward, token blocks
@@ -1141,7 +1283,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_block_kernel(const BwdArgs
   const float scale = a.scale;
   int phase = 0;
 
-  fill_query_lds<G, CH>(a.query, q_lds, tail0, D, R);
+  fill_query_lds<G, CH, VEC>(a.query, q_lds, tail0, D, R);
   float dq[CH][kVec];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
@@ -1278,7 +1420,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_block_kernel(const BwdArgs
     }
   }
 
-  store_dq_partial<G, CH>(dq, dq_lds, a.partial + static_cast<int64_t>(blockIdx.x) * R, group, lane, tail0, D);
+  store_dq_partial<G, CH, VEC>(dq, dq_lds, a.partial + static_cast<int64_t>(blockIdx.x) * R, group, lane, tail0, D);
 }
 
 // ------------------------------------------------ backward, recompute policy
@@ -1308,9 +1450,9 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_recompute_kernel(const Bwd
   const float scale = a.scale;
   int phase = 0;
 
-  fill_query_lds<G, CH>(a.query, q_lds, tail0, D, R);
+  fill_query_lds<G, CH, VEC>(a.query, q_lds, tail0, D, R);
   uint32_t km[CH][4];
-  if constexpr (!NOMASK) key_masks<G, CH>(lane, D, tail0, km);
+  if constexpr (!NOMASK) key_masks<G, CH, VEC>(lane, D, tail0, km);
   float dq[CH][kVec];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
@@ -1336,7 +1478,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_recompute_kernel(const Bwd
     }
     const float run_max = a.stats[token];
     const float inv_sum = a.stats[a.n_tokens + token];
-    if constexpr (!NOMASK) mask_range<G, CH>(lane, D, g);
+    if constexpr (!NOMASK) mask_range<G, CH, VEC>(lane, D, g);
 
     float dw[SM];
 #pragma unroll
@@ -1395,7 +1537,7 @@ __global__ void __launch_bounds__(kBlock) attnres_bwd_recompute_kernel(const Bwd
       }
     }
   }
-  store_dq_partial<G, CH>(dq, dq_lds, a.partial + static_cast<int64_t>(blockIdx.x) * R, group, lane, tail0, D);
+  store_dq_partial<G, CH, VEC>(dq, dq_lds, a.partial + static_cast<int64_t>(blockIdx.x) * R, group, lane, tail0, D);
 }
 
 // ------------------------------------------- backward, key-resident (R < D)
@@ -1754,7 +1896,7 @@ __global__ void __launch_bounds__(kBlock) attnres_gather_kernel(const GatherArgs
         const uint32_t vw[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const int d = d0 + 2 * k;
+          const int d = chunk_pos<VEC>(d0, D) + 2 * k;
           acc[t][c][2 * k] = fmaf(d >= a.tail0 ? bsum[t] : 0.0f, bf16_lo(vw[k]), acc[t][c][2 * k]);
           acc[t][c][2 * k + 1] = fmaf(d + 1 >= a.tail0 ? bsum[t] : 0.0f, bf16_hi(vw[k]), acc[t][c][2 * k + 1]);
         }
@@ -1768,21 +1910,9 @@ __global__ void __launch_bounds__(kBlock) attnres_gather_kernel(const GatherArgs
         float* grad_row = static_cast<float*>(a.grad) + tok[t] * D;
         if (a.accumulate) {  // uniform
 #pragma unroll
-          for (int e = 0; e < kVec; ++e) acc[t][c][e] += grad_row[min(d0 + e, D - 1)];
+          for (int e = 0; e < kVec; ++e) acc[t][c][e] += grad_row[min(chunk_pos<VEC>(d0, D) + e, D - 1)];
         }
-        if constexpr (VEC) {
-          if (d0 < D) {
-            __builtin_nontemporal_store(f32x4{acc[t][c][0], acc[t][c][1], acc[t][c][2], acc[t][c][3]},
-                                        reinterpret_cast<f32x4*>(grad_row + d0));
-            __builtin_nontemporal_store(f32x4{acc[t][c][4], acc[t][c][5], acc[t][c][6], acc[t][c][7]},
-                                        reinterpret_cast<f32x4*>(grad_row + d0 + 4));
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < kVec; ++e) {
-            if (d0 + e < D) grad_row[d0 + e] = acc[t][c][e];
-          }
-        }
+        if (d0 < D) store_chunk_f32<VEC>(grad_row, d0, D, acc[t][c]);
       }
     }
   }
