@@ -829,6 +829,283 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_block_kernel(const FwdArgs
   }
 }
 
+// ----------------------------------------------------- forward, few tokens
+
+// Few tokens leave the streaming forwards to latency: a group walks its
+// token's S rows one after another with at most four in flight, so one token
+// of 25 rows took 43 us, a dozen trips to memory, on one of 256 CUs.  This
+// kernel gives a token a workgroup of up to 1024 threads and takes two trips:
+//   1. every token group of the workgroup (the geometry's G lanes) takes rows
+//      g, g + groups, ... and forms their logits;
+//   2. with all logits known, the softmax's running maxima are a prefix
+//      maximum, so each source's rescale factor and weight are formed at once;
+//      then every thread owns a few columns and adds the rows, which the first
+//      trip left in L2 (the first batch is requested before the logits).
+// The sums are the streaming kernels', lane for lane and source by source
+// (same dot2 chains and lane sums; acc * alpha + w * v with the same alpha and
+// w, where alpha = 1 leaves acc as it is), so the results are bit-identical: a
+// token's output does not depend on how many others are read with it.
+constexpr int few_threads(int chunks) { return chunks == 8 ? 512 : 1024; }  // registers: 256 or 128 per thread
+
+// Columns per thread of the second trip, as few as the threads allow down to
+// 4 bytes per load (D = 1024, one token of 48 sources, 4 -> 2 columns: 9.3 -> 8.1
+// us; D = 2048, S = 48, 8 -> 4: 12.2 -> 9.9, but 4 -> 2: 9.4 -> 10.1).
+constexpr int few_columns(int lanes, int chunks) {
+  return lanes * chunks >= 512 ? 8 : lanes * chunks == 256 ? 4 : 2;
+}
+
+// EPT consecutive elements at e0 (the thread's own start) as packed words.  An
+// unaligned row's last words are moved back over the words before, as
+// load_row's last chunk is; with two columns its last element is repeated.
+template <int EPT, bool VEC>
+__device__ __forceinline__ void load_columns(const uint16_t* row, int e0, int D, uint32_t (&w)[EPT / 2]) {
+  if constexpr (EPT == 2) {
+    if constexpr (VEC) {
+      w[0] = *reinterpret_cast<const uint32_t*>(row + min(e0, D - 2));
+    } else {
+      w[0] = row[min(e0, D - 1)] | (static_cast<uint32_t>(row[min(e0 + 1, D - 1)]) << 16);
+    }
+  } else if constexpr (EPT == 4) {
+    const u32x2 x = VEC ? *reinterpret_cast<const u32x2*>(row + min(e0, D - EPT))
+                        : static_cast<u32x2>(*reinterpret_cast<const u32x2_at2*>(row + min(e0, D - EPT)));
+    w[0] = x.x, w[1] = x.y;
+  } else {
+    const u32x4 x = VEC ? *reinterpret_cast<const u32x4*>(row + min(e0, D - EPT))
+                        : static_cast<u32x4>(*reinterpret_cast<const u32x4_at2*>(row + min(e0, D - EPT)));
+    w[0] = x.x, w[1] = x.y, w[2] = x.z, w[3] = x.w;
+  }
+}
+
+// Inclusive prefix maximum over the wavefront's lanes (NaN counts as -inf):
+// row shifts inside each 16-lane row, then the rows' last lanes.
+__device__ __forceinline__ float wave_prefix_max(float x) {
+  x = fmaxf(x, -INFINITY);
+  // lanes that would shift in from outside their row keep -inf
+  auto shifted = [](float v, auto ctrl) __attribute__((always_inline)) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(-INFINITY), __float_as_int(v), ctrl.value, 0xf, 0xf,
+                                                      false));
+  };
+  x = fmaxf(x, shifted(x, std::integral_constant<int, 0x111>{}));  // row_shr:1
+  x = fmaxf(x, shifted(x, std::integral_constant<int, 0x112>{}));  // row_shr:2
+  x = fmaxf(x, shifted(x, std::integral_constant<int, 0x114>{}));  // row_shr:4
+  x = fmaxf(x, shifted(x, std::integral_constant<int, 0x118>{}));  // row_shr:8
+  const int row = (threadIdx.x & 63) / 16;
+  const float r0 = lane_value(x, 15), r1 = fmaxf(r0, lane_value(x, 31)), r2 = fmaxf(r1, lane_value(x, 47));
+  return fmaxf(x, row == 0 ? -INFINITY : row == 1 ? r0 : row == 2 ? r1 : r2);
+}
+
+// The value of the lane before; `first` in lane 0.
+__device__ __forceinline__ float wave_shift_up(float x, float first) {
+  const float before = __shfl_up(x, 1);
+  return (threadIdx.x & 63) == 0 ? first : before;
+}
+
+template <int G, int CH, bool VEC, class Rows>
+__global__ void __launch_bounds__(few_threads(CH)) attnres_fwd_few_kernel(const FwdArgs<Rows> a) {
+  constexpr int kRing = 2;                          // rows in flight per group
+  constexpr int EPT = few_columns(G, CH);           // columns per thread
+  constexpr int kBatch = EPT == 8 ? 4 : 8;          // sources per batch of the second trip
+  constexpr int kWords = G * CH * 4;                // packed words of a full row
+  constexpr int kMaxWaves = few_threads(CH) / 64;
+  __shared__ __attribute__((aligned(16))) uint32_t q_words[kWords];  // query and key masks by row position
+  __shared__ __attribute__((aligned(16))) uint32_t k_masks[kWords];
+  __shared__ float logits[kMaxSources];
+  __shared__ f32x2 steps[kMaxSources];  // alpha, w per source
+  __shared__ float xred[2][kMaxWaves][2];
+  const int threads = blockDim.x;
+  const int lane = threadIdx.x % G;
+  const int group = group_index<G>();
+  const int groups = threads / G;
+  const int D = a.width;
+  const int R = a.rank;
+  const int tail0 = D - R;
+  const int S = a.n_sources;
+  const int64_t token = blockIdx.x;
+  const float inv_R = 1.0f / static_cast<float>(R);
+
+  // Rows past S repeat row S - 1 (every lane loads, no result is used).
+  u32x4 ring[kRing][CH];
+  auto request = [&](int j, int s) __attribute__((always_inline)) {
+    const uint16_t* row = a.src.row(s < S ? s : S - 1, token);
+    if constexpr (!VEC && G == 16) {
+      load_row<G, CH, VEC>(row, lane, D, ring[j]);
+    } else {
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const int d0 = chunk_start<G>(c, lane);
+        if constexpr (VEC) {
+          ring[j][c] = *reinterpret_cast<const u32x4*>(row + (d0 < D ? d0 : 0));
+        } else {
+          ring[j][c] = *reinterpret_cast<const u32x4_at2*>(row + chunk_pos<VEC>(d0, D));
+        }
+      }
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < kRing; ++j) {
+    if (j * groups < S) request(j, group + j * groups);  // uniform
+  }
+  for (int i = threadIdx.x; i < kWords; i += threads) {
+    const int d = element_at<VEC>(2 * i, D), d1 = element_at<VEC>(2 * i + 1, D);
+    const uint32_t mask = ((d >= tail0 && d < D) ? 0x0000ffffu : 0u) | ((d1 >= tail0 && d1 < D) ? 0xffff0000u : 0u);
+    const uint32_t lo = a.query[min(max(d - tail0, 0), R - 1)];
+    const uint32_t hi = a.query[min(max(d1 - tail0, 0), R - 1)];
+    q_words[i] = (lo | (hi << 16)) & mask;
+    k_masks[i] = mask;
+  }
+  // the first batch of the second trip, on its way with the first trip
+  const int e0 = threadIdx.x * EPT;
+  uint32_t cols[kBatch][EPT / 2];
+#pragma unroll
+  for (int b = 0; b < kBatch; ++b) load_columns<EPT, VEC>(a.src.row(b < S ? b : S - 1, token), e0, D, cols[b]);
+  __syncthreads();
+
+  auto logit = [&](int j, int s, int phase) __attribute__((always_inline)) {
+    float red[2] = {0.0f, 0.0f};  // key sum of squares, <key, q>: the streaming kernels' chains
+    float ss1 = 0.0f, qd1 = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const uint32_t w[4] = {ring[j][c].x, ring[j][c].y, ring[j][c].z, ring[j][c].w};
+      const u32x4 qv = *reinterpret_cast<const u32x4*>(&q_words[(c * G + lane) * 4]);
+      const u32x4 kv = *reinterpret_cast<const u32x4*>(&k_masks[(c * G + lane) * 4]);
+      const uint32_t qw[4] = {qv.x, qv.y, qv.z, qv.w}, km[4] = {kv.x, kv.y, kv.z, kv.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t kw = w[k] & km[k];
+        if (k & 1) {
+          ss1 = dot2(kw, kw, ss1);
+          qd1 = dot2(kw, qw[k], qd1);
+        } else {
+          red[0] = dot2(kw, kw, red[0]);
+          red[1] = dot2(kw, qw[k], red[1]);
+        }
+      }
+    }
+    red[0] += ss1;
+    red[1] += qd1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) red[i] = wave_sum<(G < 64 ? G : 64)>(red[i]);
+    if constexpr (G > 64) {  // the group's waves meet in LDS, in group_sum's order
+      constexpr int kWaves = G / 64;
+      const int wave = threadIdx.x / 64;
+      if ((threadIdx.x & 63) == 0) {
+        xred[phase][wave][0] = red[0];
+        xred[phase][wave][1] = red[1];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float t = xred[phase][group * kWaves][i];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) t += xred[phase][group * kWaves + w][i];
+        red[i] = t;
+      }
+    }
+    const float inv_rms = rsqrtf(fmaf(red[0], inv_R, a.eps));
+    const float z = red[1] * inv_rms * a.scale;
+    if (lane == 0 && s < S) {
+      logits[s] = z;
+      a.logit[token * S + s] = z;
+      a.inv_rms[token * S + s] = inv_rms;
+    }
+  };
+  // rounds of one row per group; every thread takes the same number (barriers)
+  int phase = 0;
+  for (int first = 0; first < S; first += kRing * groups) {
+#pragma unroll
+    for (int j = 0; j < kRing; ++j) {
+      const int base = first + j * groups;
+      if (base < S) {  // uniform
+        logit(j, base + group, phase);
+        phase ^= 1;
+        const int next = base + kRing * groups;
+        if (next < S) request(j, next + group);  // uniform
+      }
+    }
+  }
+  __syncthreads();
+
+  // Per source: the factor its (possible) new maximum rescales the sum by, and
+  // its weight under the maximum so far.  The first wavefront scans 64 sources
+  // at a time (a NaN logit raises no maximum, as in the streaming kernels).
+  if (threadIdx.x < 64) {
+    float carry = -INFINITY;  // maximum of the sources before this round
+    for (int base = 0; base < S; base += 64) {
+      const int s = base + threadIdx.x;
+      const float z = s < S ? logits[s] : -INFINITY;
+      const float upto = fmaxf(wave_prefix_max(z), carry);  // maximum of the sources up to s
+      const float before = fmaxf(wave_shift_up(upto, carry), carry);
+      const bool raises = z > before;
+      if (s < S) steps[s] = f32x2{raises ? __expf(before - z) : 1.0f, __expf(z - (raises ? z : before))};
+      carry = lane_value(upto, 63);
+    }
+    if (threadIdx.x == 0) a.stats[token] = carry;
+  }
+  __syncthreads();
+  if (e0 >= D) return;  // no barrier follows
+
+  float acc[EPT];
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) acc[e] = 0.0f;
+  float run_sum = 0.0f;
+  auto add = [&](int b, const f32x2 step) __attribute__((always_inline)) {
+    {
+#pragma clang fp contract(off)  // the streaming kernels round the product, then the sum
+      run_sum = run_sum * step.x;
+      run_sum = run_sum + step.y;
+    }
+#pragma unroll
+    for (int k = 0; k < EPT / 2; ++k) {
+      acc[2 * k] = fmaf(step.y, bf16_lo(cols[b][k]), acc[2 * k] * step.x);
+      acc[2 * k + 1] = fmaf(step.y, bf16_hi(cols[b][k]), acc[2 * k + 1] * step.x);
+    }
+  };
+  // Whole batches refill every slot (past the last source with its row again),
+  // so no branch makes the compiler wait for the loads in flight.
+  const int rounds = S / kBatch;
+  for (int r = 0; r < rounds; ++r) {
+    f32x2 step[kBatch];
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) step[b] = steps[r * kBatch + b];
+#pragma unroll
+    for (int b = 0; b < kBatch; ++b) {
+      const int s = r * kBatch + b;
+      add(b, step[b]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_columns<EPT, VEC>(a.src.row(s + kBatch < S ? s + kBatch : S - 1, token), e0, D, cols[b]);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < kBatch; ++b) {
+    if (rounds * kBatch + b < S) add(b, steps[rounds * kBatch + b]);  // uniform
+  }
+  const float inv_sum = 1.0f / run_sum;
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) acc[e] *= inv_sum;
+
+  // Plain stores: the next kernels of a decoding step read these rows.
+  uint16_t* out = a.out + token * D;
+  int8_t* refine = a.out_refine ? a.out_refine + token * D : nullptr;
+  const int at = EPT == 2 ? e0 : min(e0, D - EPT);
+#pragma unroll
+  for (int k = 0; k < EPT / 2; ++k) {
+    const uint32_t pair = pack_bf16x2(acc[2 * k], acc[2 * k + 1]);
+    const int d = at + 2 * k;
+    if (VEC) {
+      *reinterpret_cast<uint32_t*>(out + d) = pair;
+    } else {
+      if (d >= e0 && d < D) out[d] = static_cast<uint16_t>(pair & 0xffffu);
+      if (d + 1 >= e0 && d + 1 < D) out[d + 1] = static_cast<uint16_t>(pair >> 16);
+    }
+    if (refine) {
+      const int q0 = refine_encode(acc[2 * k], pair & 0xffffu), q1 = refine_encode(acc[2 * k + 1], pair >> 16);
+      if (d >= e0 && d < D) refine[d] = static_cast<int8_t>(q0);
+      if (d + 1 >= e0 && d + 1 < D) refine[d + 1] = static_cast<int8_t>(q1);
+    }
+  }
+  if (threadIdx.x == 0) a.stats[a.n_tokens + token] = inv_sum;
+}
+
 // ----------------------------------------------------------------- backward
 
 // What the backward needs per token besides the value rows: dO (packed BF16),
@@ -2086,6 +2363,37 @@ template <int G, int CH, bool NOMASK, bool VEC>
 constexpr bool kFwdBlock32x4Variant = G == 32 && CH == 4 && !NOMASK && VEC;
 constexpr int kFwdBlockShort32MinSources = 9;
 
+// Few tokens take one workgroup per token (attnres_fwd_few_kernel): at most one
+// per CU, and two for rows of up to 2048 elements.  A workgroup of up to 1024
+// threads has a CU nearly to itself, so past that the tokens queue while the
+// streaming kernels still hide their latency; wider rows move enough bytes per
+// token to get there sooner.  Measured on MI355X (no-grad forwards in a
+// replayed graph, us per read, streaming -> this): one token, S = 25: D = 2048:
+// 44.0 -> 7.3, D = 1024: 17.4 -> 5.4, D = 4096: 36.3 -> 10.9; S = 2, D = 1024:
+// 4.4 -> 3.7; 16 tokens, S = 48, D = 1024: 32.0 -> 8.0; 256 tokens: S = 25,
+// D = 2048: 56.9 -> 11.8, S = 9, D = 8192: 21.7 -> 18.0, S = 25, D = 256: 19.2
+// -> 7.8; 512 tokens: S = 25, D = 1024: 19.5 -> 13.7, S = 48, D = 2048: 35.4 ->
+// 32.2, S = 3: 6.6 -> 6.5; but S = 9, D = 4096: 16.3 -> 19.8, D = 8192: 23.5 ->
+// 33.5, and 1024 tokens, S = 25, D = 1024: 20.2 -> 35.  Reads of one source
+// have no second row to wait for and keep the streaming kernel.
+inline bool few_tokens(int64_t n_tokens, int width) {
+  const int64_t cus = device_cus();
+  return n_tokens <= (width <= 2048 ? 2 * cus : cus);
+}
+
+template <int G, int CH, bool VEC, class Rows>
+bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
+  if (a.n_sources < 2 || !few_tokens(a.n_tokens, a.width)) return false;
+  constexpr int kColumnThreads = G * CH * kVec / few_columns(G, CH);
+  int threads = (a.n_sources * G + 63) / 64 * 64;
+  if (threads < kColumnThreads) threads = kColumnThreads;
+  if (threads < kBlock) threads = kBlock;
+  if (threads > few_threads(CH)) threads = few_threads(CH);
+  hipLaunchKernelGGL((attnres_fwd_few_kernel<G, CH, VEC, Rows>), dim3(static_cast<unsigned>(a.n_tokens)),
+                     dim3(static_cast<unsigned>(threads)), 0, stream, a);
+  return true;
+}
+
 template <int G, int CH, bool NOMASK, bool VEC, class Rows>
 void launch_fwd(const FwdArgs<Rows>& a, hipStream_t stream) {
   constexpr int64_t kGroups = kBlock / G;
@@ -2141,6 +2449,7 @@ extern template void launch_fwd<64, 8, false, false, ListRows>(const FwdArgs<Lis
 
 template <int G, int CH, class Rows>
 void launch_fwd_geometry(const FwdArgs<Rows>& a, bool nomask, bool vec, hipStream_t stream) {
+  if (vec ? launch_fwd_few<G, CH, true>(a, stream) : launch_fwd_few<G, CH, false>(a, stream)) return;
   if (nomask) {
     if (vec) launch_fwd<G, CH, true, true>(a, stream);
     else launch_fwd<G, CH, true, false>(a, stream);
