@@ -40,7 +40,7 @@ OUTPUT = HERE / "attnres" / "_lib" / "libattnres_hip.so"
 ARCH = "gfx950"
 # (lanes, chunks) per translation unit; must match ATTNRES_FOR_EACH_GEOMETRY
 # in csrc/attnres_internal.h.
-GEOMETRIES = ((16, 1), (32, 1), (32, 2), (32, 4), (64, 4), (64, 8), (256, 4))
+GEOMETRIES = ((16, 1), (32, 1), (32, 2), (32, 3), (32, 4), (64, 3), (64, 4), (64, 5), (64, 6), (64, 8), (256, 3), (256, 4))
 # geometries built as two units (ATTNRES_UNIT_PART 1: forwards and gather;
 # 2: backwards, and for (64, 8) the masked forwards), with extra flags for
 # part 2: the (64, 8) backwards (streaming, key-resident, recompute) are

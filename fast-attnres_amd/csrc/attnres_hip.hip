@@ -240,13 +240,11 @@ int launch_forward(const FwdArgs<Rows>& a, bool vec, hipStream_t stream) {
   const Geometry geo = geometry(a.width);
   const bool nomask = no_mask(geo, a.width, a.rank);
   switch (geo.lanes * 100 + geo.chunks) {
-    case 1601: launch_fwd_geometry<16, 1>(a, nomask, vec, stream); break;
-    case 3201: launch_fwd_geometry<32, 1>(a, nomask, vec, stream); break;
-    case 3202: launch_fwd_geometry<32, 2>(a, nomask, vec, stream); break;
-    case 3204: launch_fwd_geometry<32, 4>(a, nomask, vec, stream); break;
-    case 6404: launch_fwd_geometry<64, 4>(a, nomask, vec, stream); break;
-    case 6408: launch_fwd_geometry<64, 8>(a, nomask, vec, stream); break;
-    default: launch_fwd_geometry<256, 4>(a, nomask, vec, stream); break;
+#define ATTNRES_CASE(G, CH) \
+  case G * 100 + CH: launch_fwd_geometry<G, CH>(a, nomask, vec, stream); break;
+    ATTNRES_FOR_EACH_GEOMETRY(ATTNRES_CASE)
+#undef ATTNRES_CASE
+    default: break;  // not reached: geometry() returns one of the table's
   }
   return launch_status("attnres forward");
 }
@@ -286,13 +284,11 @@ int launch_backward(const BwdArgs<Rows, Grads>& a, bool vec, bool acc, bool reco
   const bool nomask = no_mask(geo, a.width, a.rank);
   int64_t blocks = 0;
   switch (geo.lanes * 100 + geo.chunks) {
-    case 1601: blocks = launch_bwd_select<16, 1>(a, nomask, vec, acc, recompute, stream); break;
-    case 3201: blocks = launch_bwd_select<32, 1>(a, nomask, vec, acc, recompute, stream); break;
-    case 3202: blocks = launch_bwd_select<32, 2>(a, nomask, vec, acc, recompute, stream); break;
-    case 3204: blocks = launch_bwd_select<32, 4>(a, nomask, vec, acc, recompute, stream); break;
-    case 6404: blocks = launch_bwd_select<64, 4>(a, nomask, vec, acc, recompute, stream); break;
-    case 6408: blocks = launch_bwd_select<64, 8>(a, nomask, vec, acc, recompute, stream); break;
-    default: blocks = launch_bwd_select<256, 4>(a, nomask, vec, acc, recompute, stream); break;
+#define ATTNRES_CASE(G, CH) \
+  case G * 100 + CH: blocks = launch_bwd_select<G, CH>(a, nomask, vec, acc, recompute, stream); break;
+    ATTNRES_FOR_EACH_GEOMETRY(ATTNRES_CASE)
+#undef ATTNRES_CASE
+    default: break;  // not reached: geometry() returns one of the table's
   }
   int st = launch_status("attnres backward");
   if (st != ATTNRES_OK) return st;
@@ -785,13 +781,11 @@ int attnres_hip_bank_gather(const void* values, int64_t row_stride, int64_t n_to
     }
     a.n_reads = count;
     switch (geo.lanes * 100 + geo.chunks) {
-      case 1601: launch_gather_geometry<16, 1>(a, vec, s); break;
-      case 3201: launch_gather_geometry<32, 1>(a, vec, s); break;
-      case 3202: launch_gather_geometry<32, 2>(a, vec, s); break;
-      case 3204: launch_gather_geometry<32, 4>(a, vec, s); break;
-      case 6404: launch_gather_geometry<64, 4>(a, vec, s); break;
-      case 6408: launch_gather_geometry<64, 8>(a, vec, s); break;
-      default: launch_gather_geometry<256, 4>(a, vec, s); break;
+#define ATTNRES_CASE(G, CH) \
+  case G * 100 + CH: launch_gather_geometry<G, CH>(a, vec, s); break;
+      ATTNRES_FOR_EACH_GEOMETRY(ATTNRES_CASE)
+#undef ATTNRES_CASE
+      default: break;  // not reached: geometry() returns one of the table's
     }
     if ((st = launch_status("attnres bank gather")) != ATTNRES_OK) return st;
     first += count;

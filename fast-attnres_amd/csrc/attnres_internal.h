@@ -181,13 +181,25 @@ struct Geometry {
 // D = 1024, S = 9: 200 -> 190 us, S = 25: 490 -> 458, S = 48: 918 -> 885;
 // D = 512, S = 25: 264 -> 255.  At D = 2048, 32 x 8 is no faster than 64 x 4
 // (it runs at occupancy 1).
+// Rows between the powers of two have geometries of their own (3, 5 or 6
+// chunks per lane), so that fewer chunks idle and fewer registers let more
+// wavefronts run.  Measured on MI355X (backward, us, the next power of two's
+// geometry -> this one): S = 9: D = 768, N = 8192: 59.2 -> 57.4; D = 1536: 107.3
+// -> 100.5; D = 2560: 210.9 -> 163.2; D = 5120: 417 -> 321; S = 25, N = 8192: D =
+// 1280: 228 -> 208, D = 3072, R = 768: 532 -> 488.  The lanes of a row, and so
+// the order of its sums, are the same.
 inline Geometry geometry(int64_t D) {
   if (D <= 16 * kVec) return {16, 1};
   if (D <= 32 * kVec) return {32, 1};
   if (D <= 64 * kVec) return {32, 2};
+  if (D <= 96 * kVec) return {32, 3};
   if (D <= 128 * kVec) return {32, 4};
+  if (D <= 192 * kVec) return {64, 3};
   if (D <= 256 * kVec) return {64, 4};
+  if (D <= 320 * kVec) return {64, 5};
+  if (D <= 384 * kVec) return {64, 6};
   if (D <= 512 * kVec) return {64, 8};
+  if (D <= 768 * kVec) return {256, 3};
   return {256, 4};
 }
 
@@ -211,7 +223,7 @@ constexpr int kKeyResFullChunks = 4;
 inline int keyres_key_chunks(int64_t D, int64_t R) {
   const Geometry geo = geometry(D);
   const int64_t column = static_cast<int64_t>(geo.lanes) * kVec;  // elements per chunk column
-  if (geo.lanes != 64 || D != geo.chunks * column || R % column != 0) return 0;
+  if (geo.lanes != 64 || (geo.chunks != 4 && geo.chunks != 8) || D != geo.chunks * column || R % column != 0) return 0;
   const int64_t kc = R / column;
   if (kc == geo.chunks) return kc == kKeyResFullChunks ? static_cast<int>(kc) : 0;  // R = D = 2048 only
   return kc <= kKeyResMaxChunks ? static_cast<int>(kc) : 0;
@@ -229,9 +241,10 @@ inline bool recomputes(int64_t S, int64_t D, int64_t R) {
 }
 
 // Lanes per token group of the recompute backward: it keeps S rows per lane,
-// so for the (64, 8) geometry (2048 < D <= 4096) it runs a whole workgroup
-// per token with 2 chunks per lane; every other geometry keeps its group.
-constexpr int recompute_lanes(int lanes, int chunks) { return lanes == 64 && chunks == 8 ? kBlock : lanes; }
+// so for 64 lanes of 5, 6 or 8 chunks (2048 < D <= 4096) it runs a whole
+// workgroup per token with 2 chunks per lane; every other geometry keeps its
+// group.
+constexpr int recompute_lanes(int lanes, int chunks) { return lanes == 64 && chunks > 4 ? kBlock : lanes; }
 
 // Grid for N tokens in groups of `group_lanes` lanes whose groups stride over
 // the tokens: one group per token at most, capped by `resident` (the
@@ -313,7 +326,7 @@ int64_t launch_bwd_geometry_f32(const BwdArgs<Rows, Grads>& a, bool nomask, bool
   extern template int64_t launch_bwd_geometry_f32<G, CH, ListRows, ListGradsF32>(                 \
       const BwdArgs<ListRows, ListGradsF32>&, bool, bool, hipStream_t);
 
-#define ATTNRES_FOR_EACH_GEOMETRY(X) X(16, 1) X(32, 1) X(32, 2) X(32, 4) X(64, 4) X(64, 8) X(256, 4)
+#define ATTNRES_FOR_EACH_GEOMETRY(X) X(16, 1) X(32, 1) X(32, 2) X(32, 3) X(32, 4) X(64, 3) X(64, 4) X(64, 5) X(64, 6) X(64, 8) X(256, 3) X(256, 4)
 
 }  // namespace attnres_hip
 

@@ -737,6 +737,26 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_block_kernel(const FwdArgs
     run_sum[t] = 0.0f;
   }
 
+  // token t is complete: normalise and store its output row
+  auto finish = [&](int t) __attribute__((always_inline)) {
+    const int64_t token = tok[t];
+    const float inv_sum = 1.0f / run_sum[t];
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int e = 0; e < kVec; ++e) acc[t][c][e] *= inv_sum;
+    if (valid[t]) {
+      if (a.out_refine) {
+        store_row_refined<G, CH, NOMASK, VEC, true>(a.out + token * D, a.out_refine + token * D, lane, D, acc[t]);
+      } else {
+        store_row_refined<G, CH, NOMASK, VEC, false>(a.out + token * D, nullptr, lane, D, acc[t]);
+      }
+      if (lane == 0) {
+        a.stats[token] = run_max[t];
+        a.stats[N + token] = inv_sum;
+      }
+    }
+  };
   auto step = [&](int j, int s, bool refill_slot) __attribute__((always_inline)) {
     const int t = j % T;
     const int64_t token = tok[t];
@@ -797,23 +817,8 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_block_kernel(const FwdArgs
       const ItemCursor at{token, sn < S ? sn : 0, 1};
       refill<G, CH, VEC>(a.src, at, sn < S, idle, lane, D, ring[j]);
     }
-    if (s == S - 1) {
-      const float inv_sum = 1.0f / run_sum[t];
-#pragma unroll
-      for (int c = 0; c < CH; ++c)
-#pragma unroll
-        for (int e = 0; e < kVec; ++e) acc[t][c][e] *= inv_sum;
-      if (valid[t]) {
-        if (a.out_refine) {
-          store_row_refined<G, CH, NOMASK, VEC, true>(a.out + token * D, a.out_refine + token * D, lane, D, acc[t]);
-        } else {
-          store_row_refined<G, CH, NOMASK, VEC, false>(a.out + token * D, nullptr, lane, D, acc[t]);
-        }
-        if (lane == 0) {
-          a.stats[token] = run_max[t];
-          a.stats[N + token] = inv_sum;
-        }
-      }
+    if constexpr (T > 1) {
+      if (s == S - 1) finish(t);
     }
   };
 
@@ -827,6 +832,7 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_block_kernel(const FwdArgs
   for (int j = 0; j < NB; ++j) {
     if (j / T < rem) step(j, full * NBT + j / T, false);
   }
+  if constexpr (T == 1) finish(0);
 }
 
 // ----------------------------------------------------- forward, few tokens
@@ -845,13 +851,13 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_block_kernel(const FwdArgs
 // (same dot2 chains and lane sums; acc * alpha + w * v with the same alpha and
 // w, where alpha = 1 leaves acc as it is), so the results are bit-identical: a
 // token's output does not depend on how many others are read with it.
-constexpr int few_threads(int chunks) { return chunks == 8 ? 512 : 1024; }  // registers: 256 or 128 per thread
+constexpr int few_threads(int chunks) { return chunks > 4 ? 512 : 1024; }  // registers: 256 or 128 per thread
 
 // Columns per thread of the second trip, as few as the threads allow down to
 // 4 bytes per load (D = 1024, one token of 48 sources, 4 -> 2 columns: 9.3 -> 8.1
 // us; D = 2048, S = 48, 8 -> 4: 12.2 -> 9.9, but 4 -> 2: 9.4 -> 10.1).
 constexpr int few_columns(int lanes, int chunks) {
-  return lanes * chunks >= 512 ? 8 : lanes * chunks == 256 ? 4 : 2;
+  return chunks > 4 || lanes * chunks > 256 ? 8 : lanes * chunks == 256 ? 4 : 2;
 }
 
 // EPT consecutive elements at e0 (the thread's own start) as packed words.  An
@@ -2220,11 +2226,11 @@ inline int64_t device_cus() {
   return cached;
 }
 
-// Backward ring depth.  One row per group, except two for aligned,
-// non-accumulating rows of 4 chunks (the variants that keep two rows without
-// spilling): at 64 lanes (D <= 2048) and 256 lanes (D > 4096) always, at
-// 32 lanes (D <= 1024) when the grid holds at most 4 wavefronts per CU, where
-// a group has a long chain of items and little else hides its latency.
+// Backward ring depth.  One row per group, except two for non-accumulating
+// rows of 3 or 4 chunks (the variants that keep two rows without spilling):
+// whole aligned rows of 4 chunks at 64 lanes (D = 2048) and 256 lanes (D = 8192)
+// always, the others when the grid holds at most 4 wavefronts per CU, where a
+// group has a long chain of items and little else hides its latency.
 // Measured on MI355X (backward, median of 8 interleaved rounds, us):
 // S=25, N=16384, D=2048: 645 -> 637; S=9, N=8192, D=8192: 492 -> 483;
 // S=25, N=2048, D=1024: 54 -> 47 (R=D), 55 -> 48 (R=256); but at N=16384,
@@ -2234,8 +2240,14 @@ inline int64_t device_cus() {
 // are 2-3% slower with them (S=25, N=16384, D=R=4096: 1273 -> 1316; with the
 // iterative-minreg scheduler of the (64, 8) backward unit too: S=25 1295.5 ->
 // 1329.5, S=13 715.1 -> 727.6, S=48 2487.9 -> 2514.9).
-template <int CH, bool VEC, bool ACC>
-constexpr bool kBwdTwoRowVariant = CH == 4 && VEC && !ACC;
+// One row per group where rows leave chunks idle or are not aligned, whatever
+// the lanes: more wavefronts then hide more than a second row does.  Two rows ->
+// one: S = 17, N = 8192, D = 5120, R = 1280 (now 256 x 3): 664 -> 550; D = 7168,
+// R = 1792: 808 -> 712; S = 9, N = 2048, D = 1800: 47.7 -> 40.5; D = 1537: 46.1 ->
+// 37.1.  Rows of 3 chunks per lane are level (D = 1536, N = 8192, S = 9: 100.7 /
+// 100.5) and take two rows only on small grids.
+template <int CH, bool ACC>
+constexpr bool kBwdTwoRowVariant = (CH == 4 || CH == 3) && !ACC;
 
 // At most 4 wavefronts per CU for N tokens of G lanes each.
 inline bool few_waves(int64_t n_tokens, int G) {
@@ -2265,17 +2277,14 @@ int64_t resident_blocks() {
   return cached;
 }
 
-// Grid shape of the forward.  Many sources: one token per group --
-// workgroups that start as others retire spread the output stores over time
-// (a persistent grid, whose groups all finish a token at once, is 2-6%
-// slower from S ~ 17 on).  Few sources: a persistent grid, whose groups
-// stream the rows of consecutive tokens through the ring without draining it
-// -- one token per group leaves a group only S rows to keep in flight before
-// it retires.  Measured on MI355X at N = 16384 (8192 for D = 8192), forward
-// time one token per group -> persistent: S = 1: 28 -> 26 us (D = 1024),
-// 59 -> 40 (2048), 144 -> 72 (4096), 110 -> 68 (8192); S = 5: 52 -> 46 (1024),
-// 98 -> 83 (2048), 227 -> 155 (4096); S = 9: 132 -> 126 (2048), 293 -> 241
-// (4096), 262 -> 249 (8192); S = 13 at D = 2048: equal; S = 17: 216 -> 224.
+// Reads of at most this many sources that take the one-token ring do so on a
+// persistent grid, whose groups stream the rows of consecutive tokens through
+// the ring without draining it: one token per group leaves a group only S rows
+// to keep in flight before it retires.  Measured on MI355X at N = 16384 (8192
+// for D = 8192), forward time one token per group -> persistent: S = 1: 28 ->
+// 26 us (D = 1024), 59 -> 40 (2048), 144 -> 72 (4096), 110 -> 68 (8192); S = 5:
+// 52 -> 46 (1024), 98 -> 83 (2048), 227 -> 155 (4096); S = 9: 293 -> 241 (4096);
+// S = 17 at D = 2048: 216 -> 224, so not beyond.
 constexpr int kPersistentFwdMaxSources = 12;
 
 template <int G, int CH, int T, int NBT, bool NOMASK, bool VEC, class Rows>
@@ -2285,83 +2294,6 @@ void launch_fwd_block(const FwdArgs<Rows>& a, hipStream_t stream) {
   hipLaunchKernelGGL((attnres_fwd_block_kernel<G, CH, T, NBT, NOMASK, VEC, Rows>), dim3(static_cast<unsigned>(blocks)),
                      dim3(kBlock), 0, stream, a);
 }
-
-// Token blocks for few sources at D = R = 2048 (aligned, unmasked): two tokens
-// per wavefront, two rows of each in flight, one block per group.  Measured on
-// MI355X (forward alone, us, persistent one-token ring -> token blocks):
-// S = 9, N = 32768: 252.7 -> 234.6; S = 12, N = 16384: 161.8 -> 152.7; S = 5,
-// N = 32768: 157.9 -> 153.4.  Four tokens of one row each were slower at these
-// S (254.6, 159.8, 176.0), and at D = 1024 (32-lane groups) the same change
-// was mixed (S = 9: 123.8 -> 118.7; S = 12, R = 256: 78.4 -> 80.1).
-constexpr int kFwdBlockMinSources = 5;
-
-// Many sources at D = R = 2048: four tokens per wavefront, one row of each in
-// flight (one wave per SIMD).  Measured on MI355X (forward alone, us, one token
-// per group -> four), after a forward / after a backward of other values:
-// S = 25, N = 16384: 319.6 -> 318.4 / 320.6 -> 299.8; S = 49, N = 8192:
-// 298.4 -> 260.4 / 298.0 -> 261.5; but S = 16: 202.0 -> 199.3 / 202.8 -> 205.4.
-// Right after the backward of the same values (a benchmark loop repeating one
-// read) the one-token forward reads part of them from the memory-side cache and
-// is as fast or faster (S = 25: 286.6 against 288.8).
-constexpr int kFwdBlock4MinSources = 24;
-
-// 64 lanes of 8 chunks (2048 < D <= 4096, 16-byte aligned rows), masked or
-// not, past the persistent range: two tokens per wavefront, one row of each
-// in flight.  Measured on MI355X (forward alone, N = 16384, us, one token per
-// group -> token blocks): D = 3072, R = D: S = 13: 336 -> 264, S = 25: 540 ->
-// 441, S = 48: 961 -> 797; D = 2560, R = 640: S = 25: 506 -> 404; D = R =
-// 4096: S = 13: 361 -> 331, S = 25: 601 -> 588, S = 48: 1061 -> 1064; D =
-// 4096, R = 1024: S = 13: 351 -> 327, S = 25: 601 -> 586, S = 48: 1059 ->
-// 1067.  Rows of fewer than 4096 elements leave some chunks of a one-token
-// group idle, and two tokens per wavefront keep more bytes in flight.  In the
-// persistent range (S <= 12) the one-token ring stays: S = 5: 135 -> 153
-// (D = 3072); two rows per token were slower everywhere.
-template <int G, int CH, bool VEC>
-constexpr bool kFwdBlock8Variant = G == 64 && CH == 8 && VEC;
-
-// 64 lanes of 4 chunks with rows shorter than 2048 (1024 < D < 2048, aligned,
-// so some chunks of a group idle), from kFwdBlockMinSources sources: the same
-// two tokens per wavefront, one row of each in flight.  Measured on MI355X
-// (forward alone, N = 16384, us, current -> token blocks): D = 1280, R = D:
-// S = 5: 61.9 -> 58.8, S = 13: 137.4 -> 109.2, S = 48: 388.3 -> 343.2;
-// D = 1536, R = D: S = 9: 100.7 -> 92.7, S = 13: 146.4 -> 124.7, S = 25:
-// 241.6 -> 229.9, S = 48: 425.1 -> 429.3; R = 384: S = 13: 140.4 -> 124.6.
-// Full rows of 2048 with key masks were mixed (R = 512: S = 13: 166.0 ->
-// 170.0, S = 48: 635.6 -> 570.0) and keep the one-token kernel.
-template <int G, int CH, bool NOMASK, bool VEC>
-constexpr bool kFwdBlockShortVariant = G == 64 && CH == 4 && !NOMASK && VEC;
-
-// Workgroup-wide token groups (256 lanes of 4 chunks, 4096 < D <= 8192,
-// aligned), from kFwdBlockMinSources sources: two tokens per workgroup, one
-// row of each in flight.  Measured on MI355X (forward alone, N = 8192, us,
-// one token -> token blocks): D = 5120, R = D: S = 5: 120.1 -> 107.4, S = 25:
-// 487.7 -> 374.4, S = 48: 872.9 -> 700.9; D = 6144, R = 1536: S = 25: 493.1 ->
-// 452.8; D = 7168, R = D: S = 9: 228.6 -> 211.0; D = R = 8192: S = 9: 247.5 ->
-// 239.4, S = 48: 1160.8 -> 1134.0; R = 2048: S = 25: 615.3 -> 622.0.  Two
-// rows per token were slower than one.
-template <int G, int CH, bool VEC>
-constexpr bool kFwdBlockWideVariant = G == kBlock && CH == 4 && VEC;
-
-// 32-lane token groups (two per wavefront), aligned rows: at 1 or 2 chunks per
-// lane (128 < D <= 512) from kFwdBlockMinSources sources, two tokens per group
-// with two rows of each in flight; at 4 chunks (512 < D < 1024, some idle) from
-// kFwdBlockShort32MinSources, one row of each.  Measured on MI355X (forward
-// alone, N = 16384, us, one token -> token blocks): D = 512, R = D: S = 5:
-// 28.3 -> 23.3, S = 25: 85.2 -> 77.7, S = 48: 153.2 -> 146.3; D = 384: S = 9:
-// 38.0 -> 30.8, S = 25: 83.0 -> 64.6, S = 48: 140.3 -> 126.2; D = 768, R = D:
-// S = 9: 53.7 -> 53.0, S = 25: 125.1 -> 111.4, S = 48: 214.1 -> 200.6; D =
-// 640, R = 160: S = 25: 115.1 -> 101.5; but S = 5: 37.2 -> 38.9 (D = 768);
-// D = 256 (1 chunk): S = 9: 24.8 -> 23.4, S = 25: 51.2 -> 45.8; D = 200: S =
-// 48: 86.6 -> 79.8.  Full rows of 1024 were within +-3% either way and keep
-// the one-token kernel (a wavefront per token instead, 64 lanes of 2 chunks,
-// four or eight tokens, was slower: S = 25, N = 16384, R = D: 153 -> 165-172,
-// S = 48: 282-290 -> 292-309; S = 13 equal), as do 16-lane groups (D <= 128: within +-1.5%) and
-// rows that are not 16-byte aligned (D = 3000, 1000, 5000: within +-1%).
-template <int G, int CH, bool VEC>
-constexpr bool kFwdBlock32NarrowVariant = G == 32 && CH <= 2 && VEC;
-template <int G, int CH, bool NOMASK, bool VEC>
-constexpr bool kFwdBlock32x4Variant = G == 32 && CH == 4 && !NOMASK && VEC;
-constexpr int kFwdBlockShort32MinSources = 9;
 
 // Few tokens take one workgroup per token (attnres_fwd_few_kernel): at most one
 // per CU, and two for rows of up to 2048 elements.  A workgroup of up to 1024
@@ -2394,32 +2326,104 @@ bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
   return true;
 }
 
+// Which forward a read of many tokens takes, by how full it makes the chip and
+// by its row geometry.  T x NBT: tokens per group and rows of each in flight
+// (attnres_fwd_block_kernel); "ring": attnres_fwd_kernel.  Bits are the same
+// whichever runs.  Measured on MI355X (no-grad forwards in a replayed graph,
+// us; R = D unless stated).
+//
+// * At most one wavefront per SIMD (few_waves): one token per group, four rows
+//   in flight, its epilogue after the loop.  Nothing but the rows in flight
+//   hides latency there, and token blocks would leave CUs empty.  Ring (or the
+//   block the read took before) -> 1 x 4, S = 25: D = 512, N = 2048: 20.9 ->
+//   14.7; D = 1024, N = 1024: 20.6 -> 17.3, N = 2048: 22.9 -> 21.4; D = 2048,
+//   N = 1024: 59.4 (4 x 1) -> 20.9; D = 2560, N = 768: 28.5 -> 21.2; D = 768,
+//   N = 2048: 35.2 (2 x 1) -> 17.1.
+// * Below four per SIMD (two where rows leave chunks idle): two tokens, two rows
+//   of each: the blocks still fill the chip and keep adjacent rows in flight.  S = 25, 1 x 4 / ring / larger
+//   block -> 2 x 2: D = 2048, N = 2048: 39.4 / 39.9 / 63.7 -> 37.1, N = 3072:
+//   - / 59.5 / 68.4 -> 59.2, but N = 4096 eager: - / - / 70.1 -> 71.2; D = 1536, N = 2048: 30.4 / 31.3 / 53.0 -> 28.7;
+//   D = 1024, N = 4096: 39.8 / 40.6 / 52.5 -> 37.6; D = 8192, N = 1024: 76.0 /
+//   77.9 / 77.0 -> 75.5.  (64, 8) groups keep the choice below (N = 2048,
+//   S = 25: 80.6 against 76.0).
+// * Beyond, by geometry (fwd_block_shape): what keeps most rows of adjacent
+//   tokens in flight without spilling, N = 16384 for D <= 2048, else 8192:
+//   - 32 lanes x 1: 1 x 4 (D = 256, S = 25: ring 52.0, 2 x 2 48.9, 1 x 4 47.6;
+//     N = 8192: 28.6 / 28.6 / 26.2);
+//   - 32 x 2 and 32 x 3: 2 x 2 (D = 512, S = 25: ring 87.7 -> 76.0; D = 640,
+//     N = 8192: ring 58.8, 2 x 1 53.0, 2 x 2 48.3);
+//   - 32 x 4, from 9 sources: 2 x 2 on whole rows (D = 1024, S = 13: ring 87.4
+//     -> 78.8, S = 25: 148.7 -> 140.0; S = 5: 39.0 -> 39.8), 2 x 1 on shorter
+//     ones (D = 896, S = 9: 50.9-54.7 against 58.0-60.8 for 2 x 2);
+//   - 64 x 3: 2 x 1 (D = 1280, N = 8192, S = 25: ring 99.1 -> 94.5);
+//   - 64 x 4: short rows 2 x 1 (D = 1792, one token -> two: 81 -> 78 at S = 13);
+//     whole rows with key masks 1 x 4 (R = 512, S = 25: ring 297 -> 282; S = 16:
+//     190 -> 177); whole rows without: 2 x 2 for 5 to 12 sources (S = 9,
+//     N = 32768: ring 252.7 -> 234.6), 1 x 4 for 13 to 23 (S = 20: 234.5 ->
+//     228.3), 4 x 1 from 24 (S = 25: 1 x 4 284.5, 4 x 1 277.8; S = 49,
+//     N = 8192, cold: 298 -> 260);
+//   - 64 x 5, 64 x 6 and 256 x 3, from 9 sources: 4 x 1 (D = 2560, S = 25: ring
+//     183.9, 2 x 1 177.4, 4 x 1 170.9; D = 3072: 215.1 / 212.7 / 209.7;
+//     D = 5120, N = 4096, S = 13: 112.3 / 106.5 / 100.9), but 256 x 3 only past
+//     12 wavefronts per SIMD (D = 5120, N = 1536, S = 25: 2 x 1 75.8, 4 x 1 85.9;
+//     N = 3072: 138.4 / 147.4);
+//   - 64 x 8, past 12 sources: 2 x 1 (D = 4096, S = 25, N = 16384: ring 601 ->
+//     588; S = 5 with two tokens instead of the persistent ring: 135 -> 153);
+//   - 256 x 4: 2 x 1 (D = 8192, N = 8192, S = 48: ring 1160.8 -> 1134.0).
+//   Reads of fewer than 5 sources stay with the persistent ring (D = 2048, S =
+//   3: ring 50, 2 x 2 54.6, 1 x 4 58.7), and so do 16-lane groups (D <= 128,
+//   within +-1.5%).
+constexpr int kFwdBlockMinSources = 5;
+
+struct FwdBlockShape {
+  int tokens;  // per group; 0: the one-token ring
+  int rows;    // of each in flight
+};
+
+inline FwdBlockShape fwd_block_shape(int G, int CH, bool whole, bool nomask, int S) {
+  if (S < kFwdBlockMinSources || G == 16) return {0, 0};
+  if (G == 32) {
+    if (CH == 1) return {1, 4};
+    if (CH < 4) return {2, 2};
+    return S < 9 ? FwdBlockShape{0, 0} : whole ? FwdBlockShape{2, 2} : FwdBlockShape{2, 1};
+  }
+  if (CH == 8) return S > kPersistentFwdMaxSources ? FwdBlockShape{2, 1} : FwdBlockShape{0, 0};
+  if (CH == 4 && G == 64 && whole) return !nomask ? FwdBlockShape{1, 4} : S <= 12 ? FwdBlockShape{2, 2} : S < 24 ? FwdBlockShape{1, 4} : FwdBlockShape{4, 1};
+  if (CH > 4 || (G == kBlock && CH == 3)) return S < 9 ? FwdBlockShape{0, 0} : FwdBlockShape{4, 1};
+  return {2, 1};
+}
+
 template <int G, int CH, bool NOMASK, bool VEC, class Rows>
 void launch_fwd(const FwdArgs<Rows>& a, hipStream_t stream) {
   constexpr int64_t kGroups = kBlock / G;
-  if constexpr (G == 64 && CH == 4 && NOMASK && VEC) {
-    if (a.n_sources >= kFwdBlockMinSources && a.n_sources <= kPersistentFwdMaxSources) {
-      return launch_fwd_block<G, CH, 2, 2, NOMASK, VEC>(a, stream);
+  if constexpr (G > 16) {
+    const int64_t cus = device_cus();
+    const bool whole = a.width == G * CH * kVec;
+    const auto below = [&](int64_t waves_per_cu) { return a.n_tokens * G < waves_per_cu * 64 * cus; };
+    FwdBlockShape shape = fwd_block_shape(G, CH, whole, NOMASK, a.n_sources);
+    if (G <= 64 && a.n_sources > 1 && few_waves(a.n_tokens, G)) {
+      shape = {1, 4};
+    } else if (CH > 1 && CH < 8 && a.n_sources >= kFwdBlockMinSources && below(whole ? 16 : 8)) {
+      shape = {2, 2};
+    } else if (G == kBlock && CH == 3 && shape.tokens == 4 && below(49)) {
+      shape = {2, 1};
     }
-    if (a.n_sources >= kFwdBlock4MinSources) return launch_fwd_block<G, CH, 4, 1, NOMASK, VEC>(a, stream);
-  }
-  if constexpr (kFwdBlock8Variant<G, CH, VEC>) {
-    if (a.n_sources > kPersistentFwdMaxSources) return launch_fwd_block<G, CH, 2, 1, NOMASK, VEC>(a, stream);
-  }
-  if constexpr (kFwdBlockWideVariant<G, CH, VEC>) {
-    if (a.n_sources >= kFwdBlockMinSources) return launch_fwd_block<G, CH, 2, 1, NOMASK, VEC>(a, stream);
-  }
-  if constexpr (kFwdBlock32NarrowVariant<G, CH, VEC>) {
-    if (a.n_sources >= kFwdBlockMinSources) return launch_fwd_block<G, CH, 2, 2, NOMASK, VEC>(a, stream);
-  }
-  if constexpr (kFwdBlock32x4Variant<G, CH, NOMASK, VEC>) {
-    if (a.n_sources >= kFwdBlockShort32MinSources && a.width < G * CH * kVec) {
-      return launch_fwd_block<G, CH, 2, 1, NOMASK, VEC>(a, stream);
+    // the shapes each geometry can get; a shape outside them does not compile in
+    constexpr bool kOne = G <= 64;
+    constexpr bool kTwoTwo = CH > 1 && CH < 8;
+    constexpr bool kTwoOne = (G == 32 && CH == 4) || (G == 64 && (CH == 3 || CH == 4 || CH == 8)) || G == kBlock;
+    constexpr bool kFour = (G == 64 && CH == 4 && NOMASK) || (G == 64 && (CH == 5 || CH == 6)) || (G == kBlock && CH == 3);
+    if constexpr (kOne) {
+      if (shape.tokens == 1) return launch_fwd_block<G, CH, 1, 4, NOMASK, VEC>(a, stream);
     }
-  }
-  if constexpr (kFwdBlockShortVariant<G, CH, NOMASK, VEC>) {
-    if (a.n_sources >= kFwdBlockMinSources && a.width < G * CH * kVec) {
-      return launch_fwd_block<G, CH, 2, 1, NOMASK, VEC>(a, stream);
+    if constexpr (kTwoTwo) {
+      if (shape.tokens == 2 && shape.rows == 2) return launch_fwd_block<G, CH, 2, 2, NOMASK, VEC>(a, stream);
+    }
+    if constexpr (kTwoOne) {
+      if (shape.tokens == 2 && shape.rows == 1) return launch_fwd_block<G, CH, 2, 1, NOMASK, VEC>(a, stream);
+    }
+    if constexpr (kFour) {
+      if (shape.tokens == 4) return launch_fwd_block<G, CH, 4, 1, NOMASK, VEC>(a, stream);
     }
   }
   int64_t blocks = (a.n_tokens + kGroups - 1) / kGroups;
@@ -2450,13 +2454,9 @@ extern template void launch_fwd<64, 8, false, false, ListRows>(const FwdArgs<Lis
 template <int G, int CH, class Rows>
 void launch_fwd_geometry(const FwdArgs<Rows>& a, bool nomask, bool vec, hipStream_t stream) {
   if (vec ? launch_fwd_few<G, CH, true>(a, stream) : launch_fwd_few<G, CH, false>(a, stream)) return;
-  if (nomask) {
-    if (vec) launch_fwd<G, CH, true, true>(a, stream);
-    else launch_fwd<G, CH, true, false>(a, stream);
-  } else {
-    if (vec) launch_fwd<G, CH, false, true>(a, stream);
-    else launch_fwd<G, CH, false, false>(a, stream);
-  }
+  if (!vec) launch_fwd<G, CH, false, false>(a, stream);  // whole unaligned rows too: masks that hold everything
+  else if (nomask) launch_fwd<G, CH, true, true>(a, stream);
+  else launch_fwd<G, CH, false, true>(a, stream);
 }
 
 // The streaming backward's grid: up to two times the workgroups that fit on
@@ -2494,6 +2494,15 @@ constexpr bool kBwdBlockVariant = G == 64 && CH == 4 && NOMASK && VEC && !ACC &&
 constexpr int kBwdBlockTokens = 4;
 constexpr int kBwdBlockMinSources = 13;
 
+// Fewer blocks of 4 tokens than give every CU a workgroup: the streaming kernel,
+// whose groups take one token at a time, then uses more of the chip.  Measured
+// on MI355X (backward in a replayed graph, us, token blocks -> streaming), S =
+// 25: N = 512: 117 -> 32, N = 1024: 123 -> 46, N = 2048: 127 -> 85, N = 3072:
+// 135 -> 121; but N = 4096: 154.5 -> 160.8, N = 8192: 298 -> 316.
+inline bool few_blocks(int64_t n_tokens, int G) {
+  return n_tokens * G < kBwdBlockTokens * kBlock * device_cus();
+}
+
 template <int G, int CH, int T, bool VEC, class Rows, class Grads>
 int64_t launch_bwd_block(const BwdArgs<Rows, Grads>& a, hipStream_t stream) {
   const int64_t resident = resident_blocks<&attnres_bwd_block_kernel<G, CH, T, VEC, Rows, Grads>>();
@@ -2525,22 +2534,21 @@ extern template int64_t launch_bwd_block<64, 4, kBwdBlockTokens, true, ListRows,
 template <int G, int CH, bool NOMASK, bool VEC, bool ACC, class Rows, class Grads>
 int64_t launch_bwd(const BwdArgs<Rows, Grads>& a, hipStream_t stream) {
   if constexpr (kBwdBlockVariant<G, CH, NOMASK, VEC, ACC, Grads>) {
-    if (a.n_sources >= kBwdBlockMinSources) return launch_bwd_block<G, CH, kBwdBlockTokens, VEC>(a, stream);
+    if (a.n_sources >= kBwdBlockMinSources && !few_blocks(a.n_tokens, G)) {
+      return launch_bwd_block<G, CH, kBwdBlockTokens, VEC>(a, stream);
+    }
   }
-  if constexpr (kBwdTwoRowVariant<CH, VEC, ACC> && G >= 64) {
-    return launch_bwd_ring<G, CH, 2, NOMASK, VEC, ACC>(a, stream);
-  } else if constexpr (kBwdTwoRowVariant<CH, VEC, ACC>) {
-    return few_waves(a.n_tokens, G) ? launch_bwd_ring<G, CH, 2, NOMASK, VEC, ACC>(a, stream)
-                                    : launch_bwd_ring<G, CH, 1, NOMASK, VEC, ACC>(a, stream);
-  } else {
-    return launch_bwd_ring<G, CH, 1, NOMASK, VEC, ACC>(a, stream);
+  if constexpr (kBwdTwoRowVariant<CH, ACC>) {
+    const bool whole = G >= 64 && CH == 4 && VEC && a.width == G * CH * kVec;
+    if (whole || few_waves(a.n_tokens, G)) return launch_bwd_ring<G, CH, 2, NOMASK, VEC, ACC>(a, stream);
   }
+  return launch_bwd_ring<G, CH, 1, NOMASK, VEC, ACC>(a, stream);
 }
 
 template <int G, int CH, bool ACC, class Rows, class Grads>
 int64_t launch_bwd_variant(const BwdArgs<Rows, Grads>& a, bool nomask, bool vec, hipStream_t stream) {
-  if (nomask) return vec ? launch_bwd<G, CH, true, true, ACC>(a, stream) : launch_bwd<G, CH, true, false, ACC>(a, stream);
-  return vec ? launch_bwd<G, CH, false, true, ACC>(a, stream) : launch_bwd<G, CH, false, false, ACC>(a, stream);
+  if (!vec) return launch_bwd<G, CH, false, false, ACC>(a, stream);
+  return nomask ? launch_bwd<G, CH, true, true, ACC>(a, stream) : launch_bwd<G, CH, false, true, ACC>(a, stream);
 }
 
 template <int G, int CH, class Rows, class Grads>
@@ -2633,7 +2641,7 @@ extern template int64_t launch_bwd_keyres_chunks<64, 4, 4, false, ListRows, List
 
 template <int G, int CH, class Rows, class Grads>
 int64_t launch_bwd_keyres(const BwdArgs<Rows, Grads>& a, bool vec, hipStream_t stream) {
-  if constexpr (G == 64 && CH > kKeyResMaxChunks) {
+  if constexpr (G == 64 && (CH == 4 || CH == 8)) {
     switch (keyres_key_chunks(a.width, a.rank)) {
       case 1: return vec ? launch_bwd_keyres_chunks<G, CH, 1, true>(a, stream)
                          : launch_bwd_keyres_chunks<G, CH, 1, false>(a, stream);
@@ -2659,14 +2667,13 @@ template <int G, int CH, class Rows, class Grads>
 int64_t launch_bwd_recompute_geometry(const BwdArgs<Rows, Grads>& a, bool nomask, bool vec, hipStream_t stream) {
   if (a.n_sources > kRecomputeMaxSources) return launch_bwd_keyres<G, CH>(a, vec, stream);
   constexpr int RG = recompute_lanes(G, CH);
-  constexpr int RCH = G * CH / RG;
-  static_assert(RG * RCH == G * CH, "same row coverage");
-  if (nomask) {
-    return vec ? launch_bwd_recompute<RG, RCH, true, true>(a, stream)
-               : launch_bwd_recompute<RG, RCH, true, false>(a, stream);
+  constexpr int RCH = (G * CH + RG - 1) / RG;
+  constexpr bool kSameRow = RG * RCH == G * CH;  // else the wider group's last chunks idle: always masked
+  if (!vec) return launch_bwd_recompute<RG, RCH, false, false>(a, stream);
+  if constexpr (kSameRow) {
+    if (nomask) return launch_bwd_recompute<RG, RCH, true, true>(a, stream);
   }
-  return vec ? launch_bwd_recompute<RG, RCH, false, true>(a, stream)
-             : launch_bwd_recompute<RG, RCH, false, false>(a, stream);
+  return launch_bwd_recompute<RG, RCH, false, true>(a, stream);
 }
 
 template <int G, int CH, class Rows, class Grads>
@@ -2709,9 +2716,8 @@ void launch_gather(const GatherArgs& a, hipStream_t stream) {
 // 64 lanes x 4 chunks took 204 VGPRs, 256 x 1 far fewer).
 template <int G, int CH>
 void launch_gather_geometry(const GatherArgs& a, bool vec, hipStream_t stream) {
-  constexpr int kLanes = G * CH <= kBlock ? G * CH : kBlock;
-  constexpr int kChunks = G * CH / kLanes;
-  static_assert(kLanes * kChunks == G * CH, "same row coverage");
+  constexpr int kLanes = G * CH > kBlock / 2 ? kBlock : G * CH > kBlock / 4 ? kBlock / 2 : G * CH > kBlock / 8 ? kBlock / 4 : G * CH;
+  constexpr int kChunks = (G * CH + kLanes - 1) / kLanes;
   if (vec) {
     if (a.bf16_out) launch_gather<kLanes, kChunks, true, true>(a, stream);
     else launch_gather<kLanes, kChunks, true, false>(a, stream);
