@@ -29,7 +29,9 @@ gradients, like the read itself.
 The autograd nodes hold the buffers and the per-pass bookkeeping in a state
 object that holds no token, so the buffers are freed with the graph, without
 waiting for Python's cycle collector (a node that held the bank itself would
-close a cycle bank -> token -> node -> bank).
+close a cycle bank -> token -> node -> bank).  A ``SourceBank``'s nodes and
+state are C++ (`csrc/attnres_autograd.cpp`): the backward of a read or a push
+runs without Python.
 
 The reference has no counterpart: its shared sources' gradients are summed
 by autograd (the Block-schedule reads of `benchmarks/model.py:306-338`).
@@ -38,18 +40,15 @@ by autograd (the Block-schedule reads of `benchmarks/model.py:306-338`).
 from __future__ import annotations
 
 import ctypes
-from array import array
 from typing import Sequence
 
 import torch
 from torch import Tensor
 
 from . import _native
-from ._ops import (_contiguous, _dq_workspace, _on_device, _source_table, _stream, packed_forward_impl,
-                   sources_forward_impl)
+from ._ops import _contiguous, _dq_workspace, _on_device, _source_table, _stream, sources_forward_impl
 from ._sources import _EPS, _MAX_SOURCES, _MAX_WIDTH, check_query, check_sources
 
-_DTYPE_F32, _DTYPE_BF16 = 0, 1  # attnres_hip.h ATTNRES_DTYPE_*
 _MAX_GATHER_READS = 48  # attnres_hip.h ATTNRES_MAX_GATHER_READS
 # A BF16 source's gathered gradient is stored as BF16 by the gather itself
 # when one launch covers its reads (else FP32, converted afterwards).
@@ -61,11 +60,6 @@ class _GatherRead(ctypes.Structure):
 
     _fields_ = [("grad_out", ctypes.c_void_p), ("query_row", ctypes.c_void_p), ("coef", ctypes.c_void_p),
                 ("n_sources", ctypes.c_int64), ("position", ctypes.c_int64), ("rank", ctypes.c_int64)]
-
-
-# A gather's read table is passed as an int64 array of the same layout (six
-# 8-byte fields per read), filled without per-field ctypes attribute writes.
-assert ctypes.sizeof(_GatherRead) == 6 * 8 and _GatherRead.position.offset == 4 * 8
 
 
 _GRAPH_TASK_ID = getattr(torch._C, "_current_graph_task_id", None)
@@ -199,155 +193,6 @@ class _Read(torch.autograd.Function):
         return None, token_grad, grad_query if ctx.needs_input_grad[2] else None, None, None
 
 
-class _BankState:
-    """The slot buffer and this pass's gradient bookkeeping, used by the
-    nodes of a ``SourceBank``."""
-
-    def __init__(self, capacity: int, gradients: str) -> None:
-        self.capacity = capacity
-        self.gradients = gradients
-        self._values: Tensor | None = None
-        self._flat: Tensor | None = None  # _values viewed as [capacity, tokens, width]
-        self._width = self._tokens = self._base = 0
-        self._device: torch.device | None = None
-        self._grads: Tensor | None = None
-        self._written: list[bool] = [False] * capacity
-        self._pending: list[list[tuple[tuple, int]]] = [[] for _ in range(capacity)]
-        self._pass = -1
-
-    def _allocate(self, source: Tensor) -> None:
-        self._values = torch.empty((self.capacity, *source.shape), device=source.device, dtype=torch.bfloat16)
-        self._width = int(source.shape[-1])
-        self._tokens = source.numel() // self._width
-        self._device = source.device
-        self._flat = self._values.view(self.capacity, self._tokens, self._width)
-        self._base = self._values.data_ptr()
-
-    def _slot_ptr(self, slot: int) -> int:
-        """Device address of slot ``slot``'s BF16 rows (the buffer is contiguous)."""
-        return self._base + slot * self._tokens * self._width * 2
-
-    def _sources(self, slots: tuple[int, ...]) -> list[Tensor]:
-        return [self._values[i] for i in slots]
-
-    def _prefix(self, slots: tuple[int, ...]) -> bool:
-        return slots == tuple(range(len(slots)))
-
-    def _backward(self, slots: tuple[int, ...], query: Tensor, out: Tensor, out_refine: Tensor, grad_out: Tensor,
-                  logit: Tensor, inv_rms: Tensor, stats: Tensor, scale: float) -> Tensor:
-        current = _pass_id()
-        if self._pass != current:
-            # first read of this pass: nothing left from an earlier pass (one that stopped short
-            # of the sources) is used, and sums handed out earlier stay valid (fresh buffers)
-            self._grads = None
-            self._written = [False] * self.capacity
-            self._pending = [[] for _ in range(self.capacity)]
-            self._pass = current
-        if self.gradients == "gather":
-            return self._backward_coef(slots, query, out, out_refine, grad_out, logit, inv_rms, stats, scale)
-        lib = _native.load()
-        count = len(slots)
-        width, tokens, device = self._width, self._tokens, self._device
-        rank = query.numel()
-        if self._grads is None:
-            self._grads = torch.empty(self._values.shape, device=device, dtype=torch.float32)
-        flags = (ctypes.c_uint8 * count)(*[1 if self._written[i] else 0 for i in slots])
-        grad_query = torch.empty((rank,), device=device, dtype=torch.bfloat16)
-        workspace = _dq_workspace(lib, tokens, width, rank, device)
-        grad_out = _contiguous(grad_out.to(torch.bfloat16))
-        saved = (_contiguous(out).data_ptr(), _contiguous(out_refine).data_ptr(), grad_out.data_ptr(),
-                 _contiguous(logit).data_ptr(), _contiguous(inv_rms).data_ptr(), _contiguous(stats).data_ptr())
-        with _on_device(device):
-            if self._prefix(slots):
-                status = lib.attnres_hip_packed_backward_accumulate_f32(
-                    self._values.data_ptr(), tokens * width, width, count, tokens, width, query.data_ptr(), rank,
-                    scale, *saved, self._grads.data_ptr(), grad_query.data_ptr(), workspace.data_ptr(),
-                    workspace.numel(), flags, _stream(device))
-            else:
-                pointers = (ctypes.c_void_p * count)(*[self._slot_ptr(i) for i in slots])
-                strides = (ctypes.c_int64 * count)(*([width] * count))
-                sums = (ctypes.c_void_p * count)(*[self._grads[i].data_ptr() for i in slots])
-                status = lib.attnres_hip_sources_backward_accumulate_f32(
-                    pointers, strides, count, tokens, width, query.data_ptr(), rank, scale, *saved, sums,
-                    grad_query.data_ptr(), workspace.data_ptr(), workspace.numel(), flags, _stream(device))
-        _native.check(status, "attnres source-bank backward")
-        for i in slots:
-            self._written[i] = True
-        return grad_query
-
-    def _backward_coef(self, slots: tuple[int, ...], query: Tensor, out: Tensor, out_refine: Tensor,
-                       grad_out: Tensor, logit: Tensor, inv_rms: Tensor, stats: Tensor, scale: float) -> Tensor:
-        """First stage of the gathered gradients: dq and the dv coefficients now;
-        the read's dO and coefficients are kept for the slots' gathers."""
-        lib = _native.load()
-        count = len(slots)
-        width, tokens, device = self._width, self._tokens, self._device
-        rank = query.numel()
-        grad_query = torch.empty((rank,), device=device, dtype=torch.bfloat16)
-        coef = torch.empty((3, count, tokens), device=device, dtype=torch.float32)
-        workspace = _dq_workspace(lib, tokens, width, rank, device)
-        grad_out = _contiguous(grad_out.to(torch.bfloat16))
-        saved = (_contiguous(out).data_ptr(), _contiguous(out_refine).data_ptr(), grad_out.data_ptr(),
-                 _contiguous(logit).data_ptr(), _contiguous(inv_rms).data_ptr(), _contiguous(stats).data_ptr())
-        with _on_device(device):
-            if self._prefix(slots):
-                status = lib.attnres_hip_packed_backward_coef(
-                    self._values.data_ptr(), tokens * width, width, count, tokens, width, query.data_ptr(), rank,
-                    scale, *saved, coef.data_ptr(), grad_query.data_ptr(), workspace.data_ptr(), workspace.numel(),
-                    _stream(device))
-            else:
-                pointers = (ctypes.c_void_p * count)(*[self._slot_ptr(i) for i in slots])
-                strides = (ctypes.c_int64 * count)(*([width] * count))
-                status = lib.attnres_hip_sources_backward_coef(
-                    pointers, strides, count, tokens, width, query.data_ptr(), rank, scale, *saved, coef.data_ptr(),
-                    grad_query.data_ptr(), workspace.data_ptr(), workspace.numel(), _stream(device))
-        _native.check(status, "attnres source-bank coefficient backward")
-        if rank == width:
-            query_row = query
-        else:  # the query is aligned to the row's last R elements, zeros before
-            query_row = torch.zeros((width,), device=device, dtype=torch.bfloat16)
-            query_row[width - rank:] = query.reshape(-1)
-        # the tensors stay referenced until the slots' gathers are enqueued
-        record = ((grad_out, query_row, coef), (grad_out.data_ptr(), query_row.data_ptr(), coef.data_ptr(), count),
-                  rank)
-        for position, slot in enumerate(slots):
-            self._pending[slot].append((record, position))
-        return grad_query
-
-    def _take(self, slot: int, dtype: torch.dtype) -> Tensor | None:
-        """Slot `slot`'s gradient for this pass, or None: gathered (in BF16
-        when ``dtype`` is BF16 and one gather launch covers the slot's reads,
-        else FP32), or a view of the FP32 accumulated sums."""
-        if self._pass != _pass_id():
-            return None
-        if self.gradients == "accumulate":
-            if not self._written[slot]:
-                return None
-            self._written[slot] = False
-            return self._grads[slot]
-        pending, self._pending[slot] = self._pending[slot], []
-        if not pending:
-            return None
-        lib = _native.load()
-        width, tokens, device = self._width, self._tokens, self._device
-        reads = array("q")  # attnres_gather_read[len(pending)]
-        for (_, head, rank), position in pending:
-            reads.extend(head)
-            reads.append(position)
-            reads.append(rank)
-        rank0 = pending[0][0][2]
-        bf16 = (_BF16_GATHER and dtype == torch.bfloat16 and len(pending) <= _MAX_GATHER_READS
-                and all(rank == rank0 for (_, _, rank), _ in pending))
-        grad = torch.empty(self._values.shape[1:], device=device, dtype=torch.bfloat16 if bf16 else torch.float32)
-        with _on_device(device):
-            status = lib.attnres_hip_bank_gather(self._slot_ptr(slot), width, tokens, width,
-                                                 reads.buffer_info()[0], len(pending), grad.data_ptr(),
-                                                 _DTYPE_BF16 if bf16 else _DTYPE_F32, 0,
-                                                 _stream(device))
-        _native.check(status, "attnres source-bank gather")
-        return grad
-
-
 class SourceBank:
     """Sources kept in numbered slots of one packed BF16 buffer and read as
     slot lists: the residual stream of a Full- or Block-schedule model.
@@ -399,7 +244,10 @@ class SourceBank:
             raise ValueError("gradients must be 'gather' or 'accumulate'")
         self.capacity = capacity
         self.gradients = gradients
-        self._state = _BankState(capacity, gradients)
+        self._state = None  # the C++ nodes' slots (`BankState`), allocated by the first push
+        self._nodes = None
+        self._shape: torch.Size | None = None
+        self._device: torch.device | None = None
         self._pushed: list[bool] = [False] * capacity
         self._token: Tensor | None = None  # the latest push's token
 
@@ -421,12 +269,13 @@ class SourceBank:
             raise ValueError(f"slot must be an integer in 0..{self.capacity - 1}")
         if self._pushed[slot]:
             raise ValueError(f"slot {slot} already holds a source")
-        state = self._state
-        if state._values is None:
+        if self._state is None:
             if source.ndim < 1 or source.numel() == 0 or not 1 <= source.shape[-1] <= _MAX_WIDTH:
                 raise ValueError("each source must have shape [...,D]")
-            state._allocate(source)
-        elif source.shape != state._values.shape[1:] or source.device != state._values.device:
+            self._nodes = _native.load_autograd()
+            self._state = self._nodes.BankState(self.capacity, self.gradients == "gather", _BF16_GATHER, source)
+            self._shape, self._device = source.shape, source.device
+        elif source.shape != self._shape or source.device != self._device:
             raise ValueError("all source tensors must have the same logical shape and device")
         return slot
 
@@ -434,7 +283,7 @@ class SourceBank:
         """Store ``source`` (``[..., D]``, any float dtype, on the GPU) in
         ``slot`` (default: the lowest free one); returns the slot."""
         slot = self._claim(source, slot)
-        self._token = _Push.apply(self._state, slot, source, self._token)
+        self._token = self._nodes.bank_push(self._state, slot, source, self._token)
         self._pushed[slot] = True
         return slot
 
@@ -449,7 +298,7 @@ class SourceBank:
         if prev.dtype not in (torch.float32, torch.bfloat16):
             raise TypeError("push_sum supports float32 and bfloat16 tensors")
         slot = self._claim(emitted, slot)
-        partial, self._token = _PushSum.apply(self._state, slot, prev, emitted, self._token)
+        partial, self._token = self._nodes.bank_push_sum(self._state, slot, prev, emitted, self._token)
         self._pushed[slot] = True
         return partial
 
@@ -465,26 +314,16 @@ class SourceBank:
             raise ValueError("count must be a number of leading slots")
         if not all(self._pushed[:count]):
             raise ValueError("count must select pushed slots 0..count-1")
-        slots = list(range(count))
         if tail is not None:
             if isinstance(tail, bool) or not isinstance(tail, int) or not count <= tail < self.capacity \
                     or not self._pushed[tail]:
                 raise ValueError("tail must be a pushed slot after the leading ones")
-            slots.append(tail)
-        if not slots:
+        elif count == 0:
             raise ValueError("a read needs at least one source")
         # the slots were checked at their push: BF16 rows [..., D] on one device
-        state = self._state
-        eps_value, scale_value = check_query(query, state._width, state._device, eps, scale)
-        if not _needs_gradients(query, self._token):  # the forward alone: nothing saved
-            query = _contiguous(query)
-            if state._prefix(tuple(slots)):
-                out = packed_forward_impl(state._flat[:len(slots)], query, eps_value, scale_value, False, pooled=True)[0]
-            else:
-                out = sources_forward_impl(state._sources(tuple(slots)), query, eps_value, scale_value, False,
-                                           pooled=True)[0]
-            return out.reshape(state._values.shape[1:])
-        return _BankRead.apply(self._state, tuple(slots), query, eps_value, scale_value, self._token)
+        eps_value, scale_value = check_query(query, self._shape[-1], self._device, eps, scale)
+        return self._nodes.bank_read(self._state, count, -1 if tail is None else tail, query, eps_value, scale_value,
+                                     self._token)
 
 
 def _needs_gradients(query: Tensor, token: Tensor | None) -> bool:
@@ -493,82 +332,6 @@ def _needs_gradients(query: Tensor, token: Tensor | None) -> bool:
     Otherwise a read runs the forward alone, with no refinement bytes or
     saved state, and the same output bits."""
     return torch.is_grad_enabled() and (query.requires_grad or (token is not None and token.requires_grad))
-
-
-def _token_input_grad(ctx, index: int) -> Tensor | None:
-    """The zero-size gradient of a token input (None when it has none)."""
-    return torch.empty((0,), device=ctx.token_device) if ctx.needs_input_grad[index] else None
-
-
-class _Push(torch.autograd.Function):
-    """Copy a source into its slot; the new token follows ``previous`` (the
-    token of the push before, None for the first)."""
-
-    @staticmethod
-    def forward(ctx, bank: _BankState, slot: int, source: Tensor, previous: Tensor | None) -> Tensor:
-        bank._values[slot].copy_(source.detach())
-        ctx.bank, ctx.slot, ctx.dtype, ctx.token_device = bank, slot, source.dtype, source.device
-        return source.new_empty((0,))
-
-    @staticmethod
-    def backward(ctx, _token_grad):
-        grad = ctx.bank._take(ctx.slot, ctx.dtype)
-        return None, None, None if grad is None else grad.to(ctx.dtype), _token_input_grad(ctx, 3)
-
-
-class _PushSum(torch.autograd.Function):
-    """partial = prev + emitted, with its BF16 copy written into the slot by
-    the same kernel; the gradient of both inputs is that of the partial plus
-    the slot's summed read gradient."""
-
-    @staticmethod
-    def forward(ctx, bank: _BankState, slot: int, prev: Tensor, emitted: Tensor, previous: Tensor | None):
-        lib = _native.load()
-        prev, emitted = _contiguous(prev.detach()), _contiguous(emitted.detach())
-        partial = torch.empty_like(emitted)
-        dtype = _DTYPE_F32 if emitted.dtype == torch.float32 else _DTYPE_BF16
-        with _on_device(emitted.device):
-            status = lib.attnres_hip_partial_sum(prev.data_ptr(), emitted.data_ptr(), dtype, emitted.numel(),
-                                                 partial.data_ptr(), bank._slot_ptr(slot),
-                                                 _stream(emitted.device))
-        _native.check(status, "attnres partial sum")
-        ctx.bank, ctx.slot, ctx.dtype, ctx.token_device = bank, slot, emitted.dtype, emitted.device
-        return partial, emitted.new_empty((0,))
-
-    @staticmethod
-    def backward(ctx, grad_partial, _token_grad):
-        grad = ctx.bank._take(ctx.slot, ctx.dtype)
-        if grad is not None:
-            grad = grad.to(ctx.dtype) if grad_partial is None else grad_partial + grad.to(ctx.dtype)
-        else:
-            grad = grad_partial
-        return None, None, grad, grad, _token_input_grad(ctx, 4)
-
-
-class _BankRead(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, bank: _BankState, slots: tuple[int, ...], query: Tensor, eps: float, scale: float,
-                token: Tensor) -> Tensor:
-        query = _contiguous(query)
-        shape = bank._values.shape[1:]
-        if bank._prefix(slots):
-            flat = bank._flat[:len(slots)]
-            out, out_refine, logit, inv_rms, stats = packed_forward_impl(flat, query, eps, scale, True, pooled=True)
-        else:
-            out, out_refine, logit, inv_rms, stats = sources_forward_impl(bank._sources(slots), query, eps, scale,
-                                                                         True, pooled=True)
-        # always saved: the accumulating kernels read the refinement
-        ctx.bank, ctx.slots, ctx.scale = bank, slots, scale
-        ctx.token_device = token.device
-        ctx.save_for_backward(query, out, out_refine, logit, inv_rms, stats)
-        return out.reshape(shape)
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        query, out, out_refine, logit, inv_rms, stats = ctx.saved_tensors
-        grad_query = ctx.bank._backward(ctx.slots, query, out, out_refine, grad_out, logit, inv_rms, stats,
-                                        ctx.scale)
-        return None, None, grad_query if ctx.needs_input_grad[2] else None, None, None, _token_input_grad(ctx, 5)
 
 
 __all__ = ["SharedSources", "SourceBank"]

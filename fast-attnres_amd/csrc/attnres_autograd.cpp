@@ -28,6 +28,11 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <torch/csrc/autograd/graph_task.h>
+
+#include <algorithm>
+#include <memory>
+#include <mutex>
 #include <optional>
 #include <vector>
 
@@ -343,6 +348,314 @@ Tensor sources_read(const Tensor& query, double eps, double scale, const std::ve
   return SourcesRead::apply(query, eps, scale, at::TensorList(sources));
 }
 
+// ------------------------------------------------------------- source bank
+
+// The slots of a SourceBank and one backward pass's gradient bookkeeping,
+// used by the nodes below (attnres/shared.py states the scheme).  The nodes
+// hold it and it holds no token, so nothing closes a cycle.  Backward nodes
+// run without Python's lock, possibly on several threads: `mutex` guards the
+// pass's bookkeeping.
+struct BankState : public torch::CustomClassHolder {
+  // One read's gathered terms: its dO, the query on row positions and the
+  // coefficients [3, count, N]; kept until the gathers of its slots are enqueued.
+  struct Record {
+    Tensor grad_out, query_row, coef;
+    int64_t count, rank;
+  };
+  struct Pending {
+    std::shared_ptr<Record> record;
+    int64_t position;  // of the slot in the read's list
+  };
+
+  int64_t capacity;
+  bool gather;       // gradients="gather", else accumulated FP32 sums
+  bool bf16_gather;  // a BF16 source's gradient is stored as BF16 by its one gather launch
+  Tensor values;     // [capacity, ..., D] BF16
+  int64_t tokens = 0, width = 0;
+
+  std::mutex mutex;
+  int64_t pass = -1;
+  Tensor sums;  // [capacity, ..., D] FP32 (accumulate)
+  std::vector<char> written;
+  std::vector<std::vector<Pending>> pending;
+
+  BankState(int64_t capacity_, bool gather_, bool bf16_gather_, const Tensor& source)
+      : capacity(capacity_), gather(gather_), bf16_gather(bf16_gather_), written(capacity_, 0), pending(capacity_) {
+    std::vector<int64_t> shape{capacity};
+    shape.insert(shape.end(), source.sizes().begin(), source.sizes().end());
+    values = bf16_empty(shape, source);
+    width = source.size(-1);
+    tokens = source.numel() / width;
+  }
+
+  char* slot_rows(int64_t slot) const { return static_cast<char*>(values.data_ptr()) + slot * tokens * width * 2; }
+
+  // The first read of a pass: nothing left from an earlier pass (one that
+  // stopped short of the sources) is used, and sums handed out earlier stay
+  // valid (fresh buffers).
+  void begin_pass() {
+    const int64_t current = torch::autograd::get_current_graph_task_id();
+    if (pass == current) return;
+    sums = Tensor();
+    std::fill(written.begin(), written.end(), 0);
+    for (auto& list : pending) list.clear();
+    pass = current;
+  }
+
+  // Slot `slot`'s gradient for this pass, or an undefined tensor: gathered (in
+  // BF16 when the source is BF16 and one launch covers the slot's reads, else
+  // FP32), or a view of the FP32 accumulated sums.
+  Tensor take(int64_t slot, at::ScalarType dtype) {
+    const std::lock_guard<std::mutex> lock(mutex);
+    if (pass != torch::autograd::get_current_graph_task_id()) return Tensor();
+    if (!gather) {
+      if (!written[slot]) return Tensor();
+      written[slot] = 0;
+      return sums.select(0, slot);
+    }
+    std::vector<Pending> reads;
+    reads.swap(pending[slot]);
+    if (reads.empty()) return Tensor();
+    std::vector<attnres_gather_read> table;
+    table.reserve(reads.size());
+    bool bf16 = bf16_gather && dtype == torch::kBFloat16 && reads.size() <= ATTNRES_MAX_GATHER_READS;
+    for (const Pending& p : reads) {
+      const Record& r = *p.record;
+      bf16 = bf16 && r.rank == reads[0].record->rank;
+      table.push_back({r.grad_out.data_ptr(), r.query_row.data_ptr(), r.coef.data_ptr<float>(), r.count, p.position,
+                       r.rank});
+    }
+    const c10::DeviceGuard guard(values.device());
+    Tensor grad = torch::empty(values.sizes().slice(1),
+                               values.options().dtype(bf16 ? torch::kBFloat16 : torch::kFloat32));
+    check(attnres_hip_bank_gather(slot_rows(slot), width, tokens, width, table.data(),
+                                  static_cast<int64_t>(table.size()), grad.data_ptr(),
+                                  bf16 ? ATTNRES_DTYPE_BF16 : ATTNRES_DTYPE_F32, 0, current_stream(values)),
+          "attnres source-bank gather");
+    return grad;
+  }
+};
+
+// Slots of a read: the leading `count`, then `tail` (-1: none).  Leading slots
+// alone, or followed by the next one, are a prefix of the packed buffer.
+struct Slots {
+  int64_t count, tail;
+  int64_t size() const { return count + (tail >= 0 ? 1 : 0); }
+  int64_t at(int64_t i) const { return i < count ? i : tail; }
+  bool prefix() const { return tail < 0 || tail == count; }
+};
+
+struct SlotTable {
+  std::vector<const void*> rows;
+  std::vector<int64_t> strides;
+  SlotTable(const BankState& bank, const Slots& slots) : strides(slots.size(), bank.width) {
+    for (int64_t i = 0; i < slots.size(); ++i) rows.push_back(bank.slot_rows(slots.at(i)));
+  }
+};
+
+void bank_forward(const BankState& bank, const Slots& slots, const Tensor& query, double eps, double scale,
+                  const Tensor& out, const StatePointers& state) {
+  const int64_t S = slots.size(), N = bank.tokens, D = bank.width, R = query.numel();
+  if (slots.prefix()) {
+    check(attnres_hip_packed_forward(bank.values.data_ptr(), N * D, D, S, N, D, query.data_ptr(), R,
+                                     static_cast<float>(eps), static_cast<float>(scale), out.data_ptr(), state.refine,
+                                     state.logit, state.inv_rms, state.stats, current_stream(bank.values)),
+          "attnres packed forward");
+  } else {
+    const SlotTable table(bank, slots);
+    check(attnres_hip_sources_forward(table.rows.data(), table.strides.data(), S, N, D, query.data_ptr(), R,
+                                      static_cast<float>(eps), static_cast<float>(scale), out.data_ptr(), state.refine,
+                                      state.logit, state.inv_rms, state.stats, current_stream(bank.values)),
+          "attnres source-list forward");
+  }
+}
+
+c10::intrusive_ptr<BankState> bank_of(AutogradContext* ctx) {
+  return c10::static_intrusive_pointer_cast<BankState>(ctx->saved_data["bank"].toCapsule());
+}
+
+// The zero-size token that orders the nodes, and its zero-size gradient.
+Tensor token_like(const Tensor& source) { return torch::empty({0}, source.options()); }
+
+// Copy a source into its slot; the new token follows `previous` (the token of
+// the push before; none for the first).
+struct BankPush : public torch::autograd::Function<BankPush> {
+  static Tensor forward(AutogradContext* ctx, const c10::intrusive_ptr<BankState>& bank, int64_t slot,
+                        const Tensor& source, const std::optional<Tensor>& previous) {
+    const c10::DeviceGuard guard(source.device());
+    bank->values.select(0, slot).copy_(source);
+    ctx->set_materialize_grads(false);
+    ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
+    ctx->saved_data["slot"] = slot;
+    ctx->saved_data["dtype"] = static_cast<int64_t>(source.scalar_type());
+    ctx->saved_data["token"] = previous.has_value();
+    return token_like(source);
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list) {
+    const auto bank = bank_of(ctx);
+    const auto dtype = static_cast<at::ScalarType>(ctx->saved_data["dtype"].toInt());
+    Tensor grad = bank->take(ctx->saved_data["slot"].toInt(), dtype);
+    if (grad.defined()) grad = grad.to(dtype);
+    const bool token = ctx->saved_data["token"].toBool();
+    return {Tensor(), Tensor(), grad, token ? torch::empty({0}, bank->values.options().dtype(dtype)) : Tensor()};
+  }
+};
+
+// partial = prev + emitted, with its BF16 copy written into the slot by the
+// same kernel; the gradient of both inputs is that of the partial plus the
+// slot's summed read gradient.
+struct BankPushSum : public torch::autograd::Function<BankPushSum> {
+  static variable_list forward(AutogradContext* ctx, const c10::intrusive_ptr<BankState>& bank, int64_t slot,
+                               const Tensor& prev, const Tensor& emitted, const std::optional<Tensor>& previous) {
+    const c10::DeviceGuard guard(emitted.device());
+    const Tensor a = prev.contiguous(), b = emitted.contiguous();
+    Tensor partial = torch::empty(b.sizes(), b.options());
+    check(attnres_hip_partial_sum(a.data_ptr(), b.data_ptr(),
+                                  b.scalar_type() == torch::kFloat32 ? ATTNRES_DTYPE_F32 : ATTNRES_DTYPE_BF16,
+                                  b.numel(), partial.data_ptr(), bank->slot_rows(slot), current_stream(b)),
+          "attnres partial sum");
+    ctx->set_materialize_grads(false);
+    ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
+    ctx->saved_data["slot"] = slot;
+    ctx->saved_data["dtype"] = static_cast<int64_t>(emitted.scalar_type());
+    ctx->saved_data["token"] = previous.has_value();
+    return {partial, token_like(emitted)};
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto bank = bank_of(ctx);
+    const auto dtype = static_cast<at::ScalarType>(ctx->saved_data["dtype"].toInt());
+    Tensor grad = bank->take(ctx->saved_data["slot"].toInt(), dtype);
+    if (grad.defined()) grad = grad.to(dtype);
+    if (grads[0].defined()) grad = grad.defined() ? grads[0] + grad : grads[0];
+    const bool token = ctx->saved_data["token"].toBool();
+    return {Tensor(), Tensor(), grad, grad, token ? torch::empty({0}, bank->values.options().dtype(dtype)) : Tensor()};
+  }
+};
+
+// A read of the bank's slots.  Always saves the refinement (its backward
+// kernels read it); the backward leaves dv to the slots' gathers, or adds it
+// to their FP32 sums.
+struct BankRead : public torch::autograd::Function<BankRead> {
+  static Tensor forward(AutogradContext* ctx, const c10::intrusive_ptr<BankState>& bank, int64_t count, int64_t tail,
+                        const Tensor& query, double eps, double scale, const Tensor& token) {
+    const Slots slots{count, tail};
+    const c10::DeviceGuard guard(bank->values.device());
+    const Tensor q = query.contiguous();
+    Tensor out = bf16_empty(bank->values.sizes().slice(1), bank->values);
+    const PoolLayout layout = pool_layout(bank->tokens, slots.size(), bank->width, true);
+    Tensor pool = torch::empty({layout.size}, bank->values.options().dtype(torch::kUInt8));
+    bank_forward(*bank, slots, q, eps, scale, out, pool_pointers(pool, layout, true));
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({q, pool, out});
+    ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
+    ctx->saved_data["count"] = count;
+    ctx->saved_data["tail"] = tail;
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["dtype"] = static_cast<int64_t>(token.scalar_type());
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    variable_list result(7);  // bank, count, tail, query, eps, scale, token
+    if (!grads[0].defined()) return result;
+    const auto bank = bank_of(ctx);
+    const Slots slots{ctx->saved_data["count"].toInt(), ctx->saved_data["tail"].toInt()};
+    const float scale = static_cast<float>(ctx->saved_data["scale"].toDouble());
+    const variable_list saved = ctx->get_saved_variables();
+    const Tensor &query = saved[0], &pool = saved[1], out = saved[2].contiguous();
+    const Tensor& like = bank->values;
+    const int64_t S = slots.size(), N = bank->tokens, D = bank->width, R = query.numel();
+    const c10::DeviceGuard guard(like.device());
+    const Tensor grad_out = grads[0].to(torch::kBFloat16).contiguous();
+    const StatePointers state = pool_pointers(pool, pool_layout(N, S, D, true), true);
+    Tensor grad_query = bf16_empty({R}, like);
+    Tensor workspace = dq_workspace(N, D, R, like);
+    const auto stream = current_stream(like);
+    const std::lock_guard<std::mutex> lock(bank->mutex);
+    bank->begin_pass();
+    if (bank->gather) {
+      Tensor coef = torch::empty({3, S, N}, like.options().dtype(torch::kFloat32));
+      if (slots.prefix()) {
+        check(attnres_hip_packed_backward_coef(like.data_ptr(), N * D, D, S, N, D, query.data_ptr(), R, scale,
+                                               out.data_ptr(), state.refine, grad_out.data_ptr(), state.logit,
+                                               state.inv_rms, state.stats, coef.data_ptr<float>(),
+                                               grad_query.data_ptr(), workspace.data_ptr<float>(), workspace.numel(),
+                                               stream),
+              "attnres source-bank coefficient backward");
+      } else {
+        const SlotTable table(*bank, slots);
+        check(attnres_hip_sources_backward_coef(table.rows.data(), table.strides.data(), S, N, D, query.data_ptr(), R,
+                                                scale, out.data_ptr(), state.refine, grad_out.data_ptr(), state.logit,
+                                                state.inv_rms, state.stats, coef.data_ptr<float>(),
+                                                grad_query.data_ptr(), workspace.data_ptr<float>(),
+                                                workspace.numel(), stream),
+              "attnres source-bank coefficient backward");
+      }
+      Tensor query_row = query;
+      if (R != D) {  // the query on the row's last R elements, zeros before
+        query_row = torch::zeros({D}, query.options());
+        query_row.narrow(0, D - R, R).copy_(query);
+      }
+      const auto record = std::make_shared<BankState::Record>(BankState::Record{grad_out, query_row, coef, S, R});
+      for (int64_t i = 0; i < S; ++i) bank->pending[slots.at(i)].push_back({record, i});
+    } else {
+      if (!bank->sums.defined()) bank->sums = torch::empty(like.sizes(), like.options().dtype(torch::kFloat32));
+      std::vector<uint8_t> flags;
+      for (int64_t i = 0; i < S; ++i) flags.push_back(bank->written[slots.at(i)] ? 1 : 0);
+      float* sums = bank->sums.data_ptr<float>();
+      if (slots.prefix()) {
+        check(attnres_hip_packed_backward_accumulate_f32(
+                  like.data_ptr(), N * D, D, S, N, D, query.data_ptr(), R, scale, out.data_ptr(), state.refine,
+                  grad_out.data_ptr(), state.logit, state.inv_rms, state.stats, sums, grad_query.data_ptr(),
+                  workspace.data_ptr<float>(), workspace.numel(), flags.data(), stream),
+              "attnres source-bank backward");
+      } else {
+        const SlotTable table(*bank, slots);
+        std::vector<float*> rows;
+        for (int64_t i = 0; i < S; ++i) rows.push_back(sums + slots.at(i) * N * D);
+        check(attnres_hip_sources_backward_accumulate_f32(
+                  table.rows.data(), table.strides.data(), S, N, D, query.data_ptr(), R, scale, out.data_ptr(),
+                  state.refine, grad_out.data_ptr(), state.logit, state.inv_rms, state.stats, rows.data(),
+                  grad_query.data_ptr(), workspace.data_ptr<float>(), workspace.numel(), flags.data(), stream),
+              "attnres source-bank backward");
+      }
+      for (int64_t i = 0; i < S; ++i) bank->written[slots.at(i)] = 1;
+    }
+    if (ctx->needs_input_grad(0)) result[3] = grad_query;
+    result[6] = torch::empty({0}, like.options().dtype(static_cast<at::ScalarType>(ctx->saved_data["dtype"].toInt())));
+    return result;
+  }
+};
+
+Tensor bank_push(const c10::intrusive_ptr<BankState>& bank, int64_t slot, const Tensor& source,
+                 const std::optional<Tensor>& previous) {
+  return BankPush::apply(bank, slot, source, previous);
+}
+
+std::tuple<Tensor, Tensor> bank_push_sum(const c10::intrusive_ptr<BankState>& bank, int64_t slot, const Tensor& prev,
+                                         const Tensor& emitted, const std::optional<Tensor>& previous) {
+  const variable_list results = BankPushSum::apply(bank, slot, prev, emitted, previous);
+  return {results[0], results[1]};
+}
+
+// No gradient wanted (grad mode off, or neither the query nor the sources --
+// through the token -- require one): the forward alone, nothing saved.
+Tensor bank_read(const c10::intrusive_ptr<BankState>& bank, int64_t count, int64_t tail, const Tensor& query,
+                 double eps, double scale, const Tensor& token) {
+  if (at::GradMode::is_enabled() && (query.requires_grad() || token.requires_grad())) {
+    return BankRead::apply(bank, count, tail, query, eps, scale, token);
+  }
+  const Slots slots{count, tail};
+  const c10::DeviceGuard guard(bank->values.device());
+  Tensor out = bf16_empty(bank->values.sizes().slice(1), bank->values);
+  StatePointers state{};
+  const Tensor scratch = statistics_scratch(bank->tokens, slots.size(), bank->values, &state);
+  bank_forward(*bank, slots, query.contiguous(), eps, scale, out, state);
+  return out;
+}
+
 std::tuple<int64_t, int64_t, int64_t> layout_of(int64_t tokens, int64_t sources, int64_t width, bool save) {
   const PoolLayout layout = pool_layout(tokens, sources, width, save);
   return {layout.head, layout.block, layout.size};
@@ -354,5 +667,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "Eager autograd nodes of the attnres read over the attnres_hip C ABI";
   m.def("packed_read", &packed_read, "packed read [S, ..., D] (eager autograd node)");
   m.def("sources_read", &sources_read, "source-list read (eager autograd node)");
+  py::class_<BankState, c10::intrusive_ptr<BankState>>(m, "BankState", "the slots of a SourceBank")
+      .def(py::init<int64_t, bool, bool, const Tensor&>())
+      .def_readonly("_values", &BankState::values);
+  m.def("bank_push", &bank_push, "copy a source into its slot; returns the new token");
+  m.def("bank_push_sum", &bank_push_sum, "partial sum of a block, stored in a slot; returns it and the new token");
+  m.def("bank_read", &bank_read, "read of leading slots and a tail slot (-1: none)");
   m.def("pool_layout", &layout_of, "(head, block, size) of the pooled saved state");
 }
