@@ -378,9 +378,12 @@ struct BankState : public torch::CustomClassHolder {
   Tensor sums;  // [capacity, ..., D] FP32 (accumulate)
   std::vector<char> written;
   std::vector<std::vector<Pending>> pending;
+  std::vector<Tensor> partial;  // FP32 sums of a slot's earlier reads (gather_block)
+  std::vector<char> wanted;     // the slot's source requires a gradient
 
   BankState(int64_t capacity_, bool gather_, bool bf16_gather_, const Tensor& source)
-      : capacity(capacity_), gather(gather_), bf16_gather(bf16_gather_), written(capacity_, 0), pending(capacity_) {
+      : capacity(capacity_), gather(gather_), bf16_gather(bf16_gather_), written(capacity_, 0), pending(capacity_),
+        partial(capacity_), wanted(capacity_, 0) {
     std::vector<int64_t> shape{capacity};
     shape.insert(shape.end(), source.sizes().begin(), source.sizes().end());
     values = bf16_empty(shape, source);
@@ -399,8 +402,28 @@ struct BankState : public torch::CustomClassHolder {
     sums = Tensor();
     std::fill(written.begin(), written.end(), 0);
     for (auto& list : pending) list.clear();
+    for (Tensor& sum : partial) sum = Tensor();
     pass = current;
   }
+
+  // A slot with many reads also forms the FP32 sums of the slots before it
+  // over the same reads, whose dO rows are then read once for all of them; the
+  // slots add what reads they get later to those sums.  Only where the reads
+  // saw these slots one position apart (a Full schedule's prefixes) and their
+  // sources want gradients.  A block writes and reads 8 bytes of sums per
+  // element and slot to save 2 per read, so it pays from about 9 reads on.
+  bool gather_block(int64_t slot, const std::vector<Pending>& reads) const {
+    if (reads.size() < kBlockReads || slot < ATTNRES_GATHER_SLOTS - 1) return false;
+    for (int64_t k = 1; k < ATTNRES_GATHER_SLOTS; ++k) {
+      const std::vector<Pending>& lower = pending[slot - k];
+      if (!wanted[slot - k] || partial[slot - k].defined() || lower.size() != reads.size()) return false;
+      for (size_t i = 0; i < reads.size(); ++i) {
+        if (lower[i].record != reads[i].record || lower[i].position != reads[i].position - k) return false;
+      }
+    }
+    return true;
+  }
+  static constexpr size_t kBlockReads = 9;
 
   // Slot `slot`'s gradient for this pass, or an undefined tensor: gathered (in
   // BF16 when the source is BF16 and one launch covers the slot's reads, else
@@ -415,23 +438,50 @@ struct BankState : public torch::CustomClassHolder {
     }
     std::vector<Pending> reads;
     reads.swap(pending[slot]);
-    if (reads.empty()) return Tensor();
+    Tensor base;
+    std::swap(base, partial[slot]);
+    if (reads.empty() || !wanted[slot]) return base;
     std::vector<attnres_gather_read> table;
     table.reserve(reads.size());
-    bool bf16 = bf16_gather && dtype == torch::kBFloat16 && reads.size() <= ATTNRES_MAX_GATHER_READS;
+    bool one_launch = reads.size() <= ATTNRES_MAX_GATHER_READS;
     for (const Pending& p : reads) {
       const Record& r = *p.record;
-      bf16 = bf16 && r.rank == reads[0].record->rank;
+      one_launch = one_launch && r.rank == reads[0].record->rank;
       table.push_back({r.grad_out.data_ptr(), r.query_row.data_ptr(), r.coef.data_ptr<float>(), r.count, p.position,
                        r.rank});
     }
+    const bool bf16 = one_launch && bf16_gather && dtype == torch::kBFloat16;
+    const int grad_dtype = bf16 ? ATTNRES_DTYPE_BF16 : ATTNRES_DTYPE_F32;
+    const auto count = static_cast<int64_t>(table.size());
     const c10::DeviceGuard guard(values.device());
-    Tensor grad = torch::empty(values.sizes().slice(1),
-                               values.options().dtype(bf16 ? torch::kBFloat16 : torch::kFloat32));
-    check(attnres_hip_bank_gather(slot_rows(slot), width, tokens, width, table.data(),
-                                  static_cast<int64_t>(table.size()), grad.data_ptr(),
-                                  bf16 ? ATTNRES_DTYPE_BF16 : ATTNRES_DTYPE_F32, 0, current_stream(values)),
+    const auto fp32 = values.options().dtype(torch::kFloat32);
+    if (!one_launch) {
+      const bool add = base.defined();
+      Tensor grad = add ? base : torch::empty(values.sizes().slice(1), fp32);
+      check(attnres_hip_bank_gather(slot_rows(slot), width, tokens, width, table.data(), count, grad.data_ptr(),
+                                    grad_dtype, add ? 1 : 0, current_stream(values)),
+            "attnres source-bank gather");
+      return grad;
+    }
+    Tensor grad = torch::empty(values.sizes().slice(1), bf16 ? values.options() : fp32);
+    const bool block = !base.defined() && gather_block(slot, reads);
+    Tensor lower;  // [slots - 1, ..., D]
+    if (block) {
+      std::vector<int64_t> shape{ATTNRES_GATHER_SLOTS - 1};
+      shape.insert(shape.end(), grad.sizes().begin(), grad.sizes().end());
+      lower = torch::empty(shape, fp32);
+    }
+    check(attnres_hip_bank_gather_slots(slot_rows(slot), width, tokens * width, block ? ATTNRES_GATHER_SLOTS : 1,
+                                        tokens, width, table.data(), count,
+                                        base.defined() ? base.data_ptr<float>() : nullptr, grad.data_ptr(), grad_dtype,
+                                        block ? lower.data_ptr<float>() : nullptr, current_stream(values)),
           "attnres source-bank gather");
+    if (block) {
+      for (int64_t k = 1; k < ATTNRES_GATHER_SLOTS; ++k) {
+        partial[slot - k] = lower.select(0, k - 1);
+        pending[slot - k].clear();
+      }
+    }
     return grad;
   }
 };
@@ -484,6 +534,7 @@ struct BankPush : public torch::autograd::Function<BankPush> {
                         const Tensor& source, const std::optional<Tensor>& previous) {
     const c10::DeviceGuard guard(source.device());
     bank->values.select(0, slot).copy_(source);
+    bank->wanted[slot] = source.requires_grad() ? 1 : 0;
     ctx->set_materialize_grads(false);
     ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
     ctx->saved_data["slot"] = slot;
@@ -515,6 +566,7 @@ struct BankPushSum : public torch::autograd::Function<BankPushSum> {
                                   b.scalar_type() == torch::kFloat32 ? ATTNRES_DTYPE_F32 : ATTNRES_DTYPE_BF16,
                                   b.numel(), partial.data_ptr(), bank->slot_rows(slot), current_stream(b)),
           "attnres partial sum");
+    bank->wanted[slot] = prev.requires_grad() || emitted.requires_grad() ? 1 : 0;
     ctx->set_materialize_grads(false);
     ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
     ctx->saved_data["slot"] = slot;

@@ -727,71 +727,128 @@ int attnres_hip_sources_backward_coef(const void* const* sources, const int64_t*
                                     dq_workspace_elems, nullptr, false, stream, coef);
 }
 
-int attnres_hip_bank_gather(const void* values, int64_t row_stride, int64_t n_tokens, int64_t width,
-                            const attnres_gather_read* reads, int64_t n_reads, void* grad, int grad_dtype,
-                            int accumulate, void* stream) {
+}  // extern "C"
+
+namespace attnres_hip {
+namespace {
+
+// The arguments both gather entries share: checked reads, and whether rows,
+// gradients and reads are 16-byte aligned.
+int check_gather(const char* name, const void* values, int64_t row_stride, int64_t n_tokens, int64_t width,
+                 const attnres_gather_read* reads, int64_t n_reads, const void* grad, int grad_dtype, bool one_launch,
+                 int64_t n_slots, bool* vec) {
   int st = check_shape(1, n_tokens, width, 1);
   if (st) return st;
-  if (!values || !reads || !grad) return fail(ATTNRES_ERR_NULL_POINTER, "null pointer argument to attnres_hip_bank_gather");
+  if (!values || !reads || !grad) return fail(ATTNRES_ERR_NULL_POINTER, "null pointer argument to %s", name);
   if (row_stride < 0) return fail(ATTNRES_ERR_STRIDE, "negative row stride");
   if (n_reads < 1) return fail(ATTNRES_ERR_SHAPE, "n_reads=%lld must be positive", (long long)n_reads);
   if (grad_dtype != ATTNRES_DTYPE_F32 && grad_dtype != ATTNRES_DTYPE_BF16)
     return fail(ATTNRES_ERR_SHAPE, "grad_dtype=%d is neither ATTNRES_DTYPE_F32 nor ATTNRES_DTYPE_BF16", grad_dtype);
-  const bool bf16_out = grad_dtype == ATTNRES_DTYPE_BF16;
-  if (bf16_out) {  // one launch, so that the sum is rounded once
+  if (one_launch) {
     bool one_rank = true;
     for (int64_t r = 1; r < n_reads; ++r) one_rank = one_rank && reads[r].rank == reads[0].rank;
-    if (accumulate || n_reads > ATTNRES_MAX_GATHER_READS || !one_rank)
+    if (n_reads > ATTNRES_MAX_GATHER_READS || !one_rank)
       return fail(ATTNRES_ERR_SHAPE,
                   "a BF16 gradient is written by one launch: accumulate=0, at most %d reads, all of one rank",
                   ATTNRES_MAX_GATHER_READS);
   }
-  bool vec = width % kVec == 0 && aligned16(values) && aligned16(grad) && (row_stride % kVec == 0 || n_tokens == 1);
+  *vec = width % kVec == 0 && aligned16(values) && aligned16(grad) && (row_stride % kVec == 0 || n_tokens == 1);
   for (int64_t r = 0; r < n_reads; ++r) {
     const attnres_gather_read& rd = reads[r];
     if (!rd.grad_out || !rd.query_row || !rd.coef)
-      return fail(ATTNRES_ERR_NULL_POINTER, "read %lld of attnres_hip_bank_gather has a null pointer", (long long)r);
+      return fail(ATTNRES_ERR_NULL_POINTER, "read %lld of %s has a null pointer", (long long)r, name);
     if ((st = check_shape(rd.n_sources, n_tokens, width, rd.rank))) return st;
-    if (rd.position < 0 || rd.position >= rd.n_sources)
-      return fail(ATTNRES_ERR_SHAPE, "read %lld: position %lld outside 0..%lld", (long long)r,
-                  (long long)rd.position, (long long)rd.n_sources - 1);
-    vec = vec && aligned16(rd.grad_out) && aligned16(rd.query_row);
-  }
-  // One launch per run of at most kMaxGatherReads reads with the same rank
-  // (in the caller's order); every launch after the first adds to grad.
-  const hipStream_t s = static_cast<hipStream_t>(stream);
-  const Geometry geo = geometry(width);
-  bool first_launch = true;
-  for (int64_t first = 0; first < n_reads;) {
-    GatherArgs a{};
-    a.values = static_cast<const uint16_t*>(values);
-    a.row_stride = row_stride;
-    a.grad = grad;
-    a.n_tokens = n_tokens;
-    a.width = static_cast<int>(width);
-    a.tail0 = static_cast<int>(width - reads[first].rank);
-    a.accumulate = (accumulate || !first_launch) ? 1 : 0;
-    a.bf16_out = bf16_out ? 1 : 0;
-    int count = 0;
-    while (first + count < n_reads && count < kMaxGatherReads && reads[first + count].rank == reads[first].rank) {
-      const attnres_gather_read& rd = reads[first + count];
-      a.read[count++] = GatherRead{static_cast<const uint16_t*>(rd.grad_out),
-                                   static_cast<const uint16_t*>(rd.query_row), rd.coef + rd.position * n_tokens,
-                                   rd.n_sources * n_tokens};
-    }
-    a.n_reads = count;
-    switch (geo.lanes * 100 + geo.chunks) {
-#define ATTNRES_CASE(G, CH) \
-  case G * 100 + CH: launch_gather_geometry<G, CH>(a, vec, s); break;
-      ATTNRES_FOR_EACH_GEOMETRY(ATTNRES_CASE)
-#undef ATTNRES_CASE
-      default: break;  // not reached: geometry() returns one of the table's
-    }
-    if ((st = launch_status("attnres bank gather")) != ATTNRES_OK) return st;
-    first += count;
-    first_launch = false;
+    if (rd.position < n_slots - 1 || rd.position >= rd.n_sources)
+      return fail(ATTNRES_ERR_SHAPE, "read %lld: position %lld outside %lld..%lld", (long long)r,
+                  (long long)rd.position, (long long)(n_slots - 1), (long long)rd.n_sources - 1);
+    *vec = *vec && aligned16(rd.grad_out) && aligned16(rd.query_row);
   }
   return ATTNRES_OK;
+}
+
+// One launch over `count` reads of one rank.
+int launch_gather(GatherArgs a, const attnres_gather_read* reads, int64_t count, bool vec, hipStream_t s) {
+  a.n_reads = static_cast<int>(count);
+  a.tail0 = static_cast<int>(a.width - reads[0].rank);
+  for (int64_t r = 0; r < count; ++r) {
+    a.read[r] = GatherRead{static_cast<const uint16_t*>(reads[r].grad_out),
+                           static_cast<const uint16_t*>(reads[r].query_row),
+                           reads[r].coef + reads[r].position * a.n_tokens, reads[r].n_sources * a.n_tokens};
+  }
+  const Geometry geo = geometry(a.width);
+  switch (geo.lanes * 100 + geo.chunks) {
+#define ATTNRES_CASE(G, CH) \
+  case G * 100 + CH: launch_gather_geometry<G, CH>(a, vec, s); break;
+    ATTNRES_FOR_EACH_GEOMETRY(ATTNRES_CASE)
+#undef ATTNRES_CASE
+    default: break;  // not reached: geometry() returns one of the table's
+  }
+  return launch_status("attnres bank gather");
+}
+
+GatherArgs gather_args(const void* values, int64_t row_stride, int64_t n_tokens, int64_t width, void* grad, bool bf16) {
+  GatherArgs a{};
+  a.values = static_cast<const uint16_t*>(values);
+  a.row_stride = row_stride;
+  a.grad = grad;
+  a.n_tokens = n_tokens;
+  a.width = static_cast<int>(width);
+  a.n_slots = 1;
+  a.bf16_out = bf16 ? 1 : 0;
+  return a;
+}
+
+}  // namespace
+}  // namespace attnres_hip
+
+extern "C" {
+
+int attnres_hip_bank_gather(const void* values, int64_t row_stride, int64_t n_tokens, int64_t width,
+                            const attnres_gather_read* reads, int64_t n_reads, void* grad, int grad_dtype,
+                            int accumulate, void* stream) {
+  const bool bf16_out = grad_dtype == ATTNRES_DTYPE_BF16;
+  bool vec = false;
+  const int st = check_gather("attnres_hip_bank_gather", values, row_stride, n_tokens, width, reads, n_reads, grad,
+                              grad_dtype, bf16_out, 1, &vec);
+  if (st) return st;
+  if (bf16_out && accumulate)
+    return fail(ATTNRES_ERR_SHAPE,
+                "a BF16 gradient is written by one launch: accumulate=0, at most %d reads, all of one rank",
+                ATTNRES_MAX_GATHER_READS);
+  // One launch per run of at most kMaxGatherReads reads with the same rank
+  // (in the caller's order); every launch after the first adds to grad.
+  for (int64_t first = 0; first < n_reads;) {
+    int64_t count = 0;
+    while (first + count < n_reads && count < kMaxGatherReads && reads[first + count].rank == reads[first].rank) ++count;
+    GatherArgs a = gather_args(values, row_stride, n_tokens, width, grad, bf16_out);
+    if (accumulate || first > 0) a.base = static_cast<const float*>(grad);
+    const int launched = launch_gather(a, reads + first, count, vec, static_cast<hipStream_t>(stream));
+    if (launched != ATTNRES_OK) return launched;
+    first += count;
+  }
+  return ATTNRES_OK;
+}
+
+int attnres_hip_bank_gather_slots(const void* values, int64_t row_stride, int64_t slot_stride, int64_t n_slots,
+                                  int64_t n_tokens, int64_t width, const attnres_gather_read* reads,
+                                  int64_t n_reads, const float* base, void* grad, int grad_dtype, float* partial,
+                                  void* stream) {
+  static const char* const kName = "attnres_hip_bank_gather_slots";
+  if (n_slots != 1 && n_slots != ATTNRES_GATHER_SLOTS)
+    return fail(ATTNRES_ERR_SHAPE, "n_slots=%lld is neither 1 nor %d", (long long)n_slots, ATTNRES_GATHER_SLOTS);
+  bool vec = false;
+  const int st = check_gather(kName, values, row_stride, n_tokens, width, reads, n_reads, grad, grad_dtype, true,
+                              n_slots, &vec);
+  if (st) return st;
+  if (n_slots > 1 && !partial) return fail(ATTNRES_ERR_NULL_POINTER, "null pointer argument to %s", kName);
+  if (slot_stride < 0) return fail(ATTNRES_ERR_STRIDE, "negative slot stride");
+  GatherArgs a = gather_args(values, row_stride, n_tokens, width, grad, grad_dtype == ATTNRES_DTYPE_BF16);
+  a.base = base;
+  a.n_slots = static_cast<int>(n_slots);
+  a.slot_stride = slot_stride;
+  a.partial = partial;
+  vec = vec && aligned16_or_null(base) && (n_slots == 1 || (aligned16(partial) && slot_stride % kVec == 0));
+  return launch_gather(a, reads, n_reads, vec, static_cast<hipStream_t>(stream));
 }
 
 int attnres_hip_partial_sum(const void* prev, const void* emitted, int dtype, int64_t n_elems, void* out,

@@ -153,16 +153,23 @@ struct GatherRead {
 
 // The reads of one launch share their query length R (key coordinates
 // tail0 = D - R .. D-1), so their b v terms add up to one scalar per token.
+// One launch gathers one slot, or kGatherSlots slots that the same reads saw
+// at consecutive positions: slot j's rows lie j * slot_stride before `values`
+// and its coefficients j planes rows (j * N elements) before the read's `p`.
+constexpr int kGatherSlots = ATTNRES_GATHER_SLOTS;
 struct GatherArgs {
   const uint16_t* values;  // the slot's [N, D] BF16 rows (row n at values + n * row_stride)
   int64_t row_stride;
-  void* grad;              // [N, D] contiguous: FP32, or BF16 when bf16_out
+  int64_t slot_stride;
+  void* grad;              // slot 0: [N, D] contiguous: FP32, or BF16 when bf16_out
+  const float* base;       // [N, D] FP32 added to slot 0's sums (may be grad itself); nullptr: none
+  float* partial;          // slots 1, 2, ...: their FP32 sums [n_slots - 1, N, D]
   int64_t n_tokens;
   int width;
   int tail0;
   int n_reads;
-  int accumulate;          // 1: add to grad (FP32 only), 0: write it
-  int bf16_out;            // 1: store the FP32 sums rounded to BF16 (one launch, no accumulate)
+  int n_slots;             // 1 or kGatherSlots
+  int bf16_out;            // 1: store slot 0's FP32 sums rounded to BF16 (one launch)
   GatherRead read[kMaxGatherReads];
 };
 

@@ -2096,13 +2096,38 @@ attnres_bwd_keyres_kernel(const BwdArgs<Rows, Grads> a) {
 // blocks), so each read's query row is loaded once per T tokens and its
 // coefficients for the T tokens are contiguous.  A ring of RING reads keeps
 // the next reads' rows in flight while one is added.
-// BF16OUT: the sums are stored rounded to BF16 (round to nearest even), for a
+// SL slots that the same reads saw share each dO row (SL x T accumulators).
+// Their 3 SL coefficients per read and token would cost as many loads as the
+// rows, so the workgroup first copies those of a tile of tokens to LDS (17
+// reads, N = 16384, D = 1024: 260 us with scalar loads instead).
+// BF16OUT: slot 0's sums are stored rounded to BF16 (round to nearest even), for a
 // BF16 source, instead of an FP32 row converted by a separate pass.
-template <int G, int CH, bool VEC, bool BF16OUT, int RING>
+
+// A coefficient.  Groups of whole wavefronts read it at a wave-uniform address
+// through scalar loads: per-lane loads of it cost an instruction each beside
+// the read's rows (12 of 17 per read at four tokens).
+template <int G>
+__device__ __forceinline__ float load_coefficient(const float* p) {
+  if constexpr (G >= 64) {
+    typedef const __attribute__((address_space(4))) float* constant_ptr;  // read-only during the launch
+    return *reinterpret_cast<constant_ptr>(reinterpret_cast<uintptr_t>(p));
+  } else {
+    return *p;
+  }
+}
+
+// Tokens per group iteration, and (SL > 1) per workgroup tile: 8, or one for
+// each of a workgroup's groups.
+template <int G, int CH, int SL>
+constexpr int gather_tokens() { return SL > 1 ? (CH == 1 && G >= 64 ? 2 : 1) : CH >= 4 ? 1 : 4 / CH; }
+template <int G>
+constexpr int gather_tile() { return kBlock / G > 8 ? kBlock / G : 8; }
+
+template <int G, int CH, bool VEC, bool BF16OUT, int RING, int SL>
 __global__ void __launch_bounds__(kBlock) attnres_gather_kernel(const GatherArgs a) {
   static_assert(kBlock % G == 0 && (G <= 64 || G % 64 == 0), "groups of whole wavefronts above 64 lanes");
-  constexpr int T = CH >= 4 ? 1 : 4 / CH;      // tokens per group iteration
-  constexpr int kRing = RING;                  // reads in flight per group (T rows each)
+  constexpr int T = gather_tokens<G, CH, SL>();  // tokens per group iteration
+  constexpr int kGatherTile = gather_tile<G>();
   constexpr int kGroups = kBlock / G;
   const int lane = threadIdx.x % G;
   const int group = group_index<G>();
@@ -2111,91 +2136,152 @@ __global__ void __launch_bounds__(kBlock) attnres_gather_kernel(const GatherArgs
   const int n_reads = a.n_reads;
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * kGroups + group;
   const int64_t groups = static_cast<int64_t>(gridDim.x) * kGroups;
-  const int64_t blocks = (N + T - 1) / T;
-  for (int64_t blk = gid; blk < blocks; blk += groups) {
+  // SL == 1: groups stride over blocks of T tokens.  SL > 1: workgroups stride
+  // over tiles, whose blocks go to the workgroup's groups in turn.
+  constexpr int kTileBlocks = kGatherTile / T;
+  static_assert(SL == 1 || kTileBlocks % kGroups == 0, "every group takes as many blocks of a tile");
+  __shared__ __attribute__((aligned(16))) float coef_lds[SL > 1 ? kMaxGatherReads * kGatherTile * 3 * SL : 1];
+  const int64_t tiles = (N + kGatherTile - 1) / kGatherTile;
+  int64_t tile = blockIdx.x;
+  const int64_t blocks = SL > 1 ? tiles * kTileBlocks : (N + T - 1) / T;
+  for (int64_t blk = SL > 1 ? tile * kTileBlocks + group : gid; blk < blocks;) {
+    if constexpr (SL > 1) {
+      if (blk == tile * kTileBlocks + group) {  // the tile's first round, the same for every group
+        __syncthreads();
+        for (int i = threadIdx.x; i < n_reads * 3 * SL * kGatherTile; i += kBlock) {
+          const int t = i % kGatherTile, term = i / kGatherTile % (3 * SL), r = i / (kGatherTile * 3 * SL);
+          const GatherRead& rd = a.read[r];
+          const int64_t n = tile * kGatherTile + t;
+          coef_lds[(r * kGatherTile + t) * 3 * SL + term] =
+              rd.p[(term / SL) * rd.plane_stride - (term % SL) * N + (n < N ? n : N - 1)];
+        }
+        __syncthreads();
+      }
+    }
     const int64_t token0 = blk * T;
     int64_t tok[T];  // clamped: a block past N re-reads the last token and stores nothing for it
 #pragma unroll
     for (int t = 0; t < T; ++t) tok[t] = token0 + t < N ? token0 + t : N - 1;
-    float acc[T][CH][kVec];
+    float acc[SL][T][CH][kVec];
+    float bsum[SL][T];
 #pragma unroll
-    for (int t = 0; t < T; ++t)
+    for (int j = 0; j < SL; ++j)
 #pragma unroll
-      for (int c = 0; c < CH; ++c)
+      for (int t = 0; t < T; ++t) {
+        bsum[j][t] = 0.0f;
 #pragma unroll
-        for (int e = 0; e < kVec; ++e) acc[t][c][e] = 0.0f;
-    float bsum[T];
+        for (int c = 0; c < CH; ++c)
 #pragma unroll
-    for (int t = 0; t < T; ++t) bsum[t] = 0.0f;
-    u32x4 g[kRing][T][CH], q[kRing][CH];
-    float cp[kRing][T], ca[kRing][T], cb[kRing][T];
+          for (int e = 0; e < kVec; ++e) acc[j][t][c][e] = 0.0f;
+      }
+    u32x4 g[RING][T][CH], q[RING][CH];
+    float cp[RING][SL][T], ca[RING][SL][T], cb[RING][SL][T];
     auto request = [&](int b, int r) __attribute__((always_inline)) {
       const GatherRead& rd = a.read[r < n_reads ? r : n_reads - 1];  // past the end: the last read again
       load_row<G, CH, VEC>(rd.qrow, lane, D, q[b]);
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         load_row<G, CH, VEC>(rd.grad_out + tok[t] * D, lane, D, g[b][t]);
-        cp[b][t] = rd.p[tok[t]];
-        ca[b][t] = rd.p[rd.plane_stride + tok[t]];
-        cb[b][t] = rd.p[2 * rd.plane_stride + tok[t]];
+        if constexpr (SL == 1) {
+          const float* p = rd.p + tok[t];
+          cp[b][0][t] = load_coefficient<G>(p);
+          ca[b][0][t] = load_coefficient<G>(p + rd.plane_stride);
+          cb[b][0][t] = load_coefficient<G>(p + 2 * rd.plane_stride);
+        } else {
+          const int at = static_cast<int>(token0 + t - tile * kGatherTile);
+          const float* lds = &coef_lds[((r < n_reads ? r : n_reads - 1) * kGatherTile + at) * 3 * SL];
+#pragma unroll
+          for (int j = 0; j < SL; ++j) {
+            cp[b][j][t] = lds[j];
+            ca[b][j][t] = lds[SL + j];
+            cb[b][j][t] = lds[2 * SL + j];
+          }
+        }
       }
     };
     auto add = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        bsum[t] += cb[b][t];
+#pragma unroll
+        for (int j = 0; j < SL; ++j) bsum[j][t] += cb[b][j][t];
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
           const uint32_t gw[4] = {g[b][t][c].x, g[b][t][c].y, g[b][t][c].z, g[b][t][c].w};
           const uint32_t qw[4] = {q[b][c].x, q[b][c].y, q[b][c].z, q[b][c].w};
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            acc[t][c][2 * k] = fmaf(ca[b][t], bf16_lo(qw[k]), fmaf(cp[b][t], bf16_lo(gw[k]), acc[t][c][2 * k]));
-            acc[t][c][2 * k + 1] =
-                fmaf(ca[b][t], bf16_hi(qw[k]), fmaf(cp[b][t], bf16_hi(gw[k]), acc[t][c][2 * k + 1]));
+          for (int j = 0; j < SL; ++j) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              float* x = acc[j][t][c];
+              x[2 * k] = fmaf(ca[b][j][t], bf16_lo(qw[k]), fmaf(cp[b][j][t], bf16_lo(gw[k]), x[2 * k]));
+              x[2 * k + 1] = fmaf(ca[b][j][t], bf16_hi(qw[k]), fmaf(cp[b][j][t], bf16_hi(gw[k]), x[2 * k + 1]));
+            }
           }
         }
       }
     };
 #pragma unroll
-    for (int j = 0; j < kRing; ++j) request(j, j);
-    for (int r = 0; r < n_reads; r += kRing) {
+    for (int j = 0; j < RING; ++j) request(j, j);
+    for (int r = 0; r < n_reads; r += RING) {
 #pragma unroll
-      for (int j = 0; j < kRing; ++j) {
+      for (int j = 0; j < RING; ++j) {
         if (r + j < n_reads) add(j);        // uniform
         __builtin_amdgcn_sched_barrier(0);  // refill the slot after its use
-        request(j, r + j + kRing);
+        request(j, r + j + RING);
       }
     }
-    // the key terms, then the earlier sum (accumulate) and the store
+    // the key terms, then the earlier sum (base) and the store
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       if (token0 + t >= N) break;  // uniform
-      u32x4 v[CH];
-      load_row<G, CH, VEC>(a.values + tok[t] * a.row_stride, lane, D, v);
 #pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const int d0 = chunk_start<G>(c, lane);
-        const uint32_t vw[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
+      for (int j = 0; j < SL; ++j) {
+        u32x4 v[CH];
+        load_row<G, CH, VEC>(a.values - j * a.slot_stride + tok[t] * a.row_stride, lane, D, v);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int d = chunk_pos<VEC>(d0, D) + 2 * k;
-          acc[t][c][2 * k] = fmaf(d >= a.tail0 ? bsum[t] : 0.0f, bf16_lo(vw[k]), acc[t][c][2 * k]);
-          acc[t][c][2 * k + 1] = fmaf(d + 1 >= a.tail0 ? bsum[t] : 0.0f, bf16_hi(vw[k]), acc[t][c][2 * k + 1]);
-        }
-        if constexpr (BF16OUT) {
-          uint16_t* grad_row = static_cast<uint16_t*>(a.grad) + tok[t] * D;
-          const u32x4 packed{pack_bf16x2(acc[t][c][0], acc[t][c][1]), pack_bf16x2(acc[t][c][2], acc[t][c][3]),
-                             pack_bf16x2(acc[t][c][4], acc[t][c][5]), pack_bf16x2(acc[t][c][6], acc[t][c][7])};
-          if (d0 < D) store_chunk<G, VEC>(grad_row, d0, D, packed);
-          continue;
-        }
-        float* grad_row = static_cast<float*>(a.grad) + tok[t] * D;
-        if (a.accumulate) {  // uniform
+        for (int c = 0; c < CH; ++c) {
+          const int d0 = chunk_start<G>(c, lane);
+          const int at = chunk_pos<VEC>(d0, D);
+          const uint32_t vw[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
+          float* x = acc[j][t][c];
 #pragma unroll
-          for (int e = 0; e < kVec; ++e) acc[t][c][e] += grad_row[min(chunk_pos<VEC>(d0, D) + e, D - 1)];
+          for (int k = 0; k < 4; ++k) {
+            const int d = at + 2 * k;
+            x[2 * k] = fmaf(d >= a.tail0 ? bsum[j][t] : 0.0f, bf16_lo(vw[k]), x[2 * k]);
+            x[2 * k + 1] = fmaf(d + 1 >= a.tail0 ? bsum[j][t] : 0.0f, bf16_hi(vw[k]), x[2 * k + 1]);
+          }
+          if (j == 0 && a.base) {  // uniform
+            const float* base = a.base + tok[t] * D;
+            if (VEC && d0 < D) {
+              const f32x4* row = reinterpret_cast<const f32x4*>(base + d0);
+              const f32x4 b0 = __builtin_nontemporal_load(row), b1 = __builtin_nontemporal_load(row + 1);
+              const float b[kVec] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+              for (int e = 0; e < kVec; ++e) x[e] += b[e];
+            } else if (!VEC) {
+#pragma unroll
+              for (int e = 0; e < kVec; ++e) x[e] += base[min(at + e, D - 1)];
+            }
+          }
+          if (BF16OUT && j == 0) {
+            uint16_t* grad_row = static_cast<uint16_t*>(a.grad) + tok[t] * D;
+            const u32x4 packed{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]),
+                               pack_bf16x2(x[6], x[7])};
+            if (d0 < D) store_chunk<G, VEC>(grad_row, d0, D, packed);
+            continue;
+          }
+          float* grad_row = (j == 0 ? static_cast<float*>(a.grad) : a.partial + (j - 1) * N * D) + tok[t] * D;
+          if (d0 < D) store_chunk_f32<VEC>(grad_row, d0, D, acc[j][t][c]);
         }
-        if (d0 < D) store_chunk_f32<VEC>(grad_row, d0, D, acc[t][c]);
+      }
+    }
+    if constexpr (SL == 1) {
+      blk += groups;
+    } else {
+      blk += kGroups;
+      if (blk >= (tile + 1) * kTileBlocks) {  // every group leaves the tile after as many blocks
+        tile += gridDim.x;
+        blk = tile * kTileBlocks + group;
       }
     }
   }
@@ -2686,13 +2772,17 @@ int64_t launch_bwd_geometry_coef(const BwdArgs<Rows, CoefSink>& a, bool nomask, 
   return launch_bwd_variant<G, CH, false>(a, nomask, vec, stream);
 }
 
-template <int G, int CH, bool VEC, bool BF16OUT, int RING>
+template <int G, int CH, bool VEC, bool BF16OUT, int RING, int SL>
 void launch_gather_ring(const GatherArgs& a, hipStream_t stream) {
   // the grid of the row geometry's token groups (the gather's own groups are
   // wider: it has no group sums and spreads a row over up to a workgroup)
-  const int64_t blocks = grid_blocks(a.n_tokens, geometry(a.width).lanes,
-                                     resident_blocks<&attnres_gather_kernel<G, CH, VEC, BF16OUT, RING>>());
-  hipLaunchKernelGGL((attnres_gather_kernel<G, CH, VEC, BF16OUT, RING>), dim3(static_cast<unsigned>(blocks)),
+  int64_t blocks = grid_blocks(a.n_tokens, geometry(a.width).lanes,
+                               resident_blocks<&attnres_gather_kernel<G, CH, VEC, BF16OUT, RING, SL>>());
+  if constexpr (SL > 1) {  // a tile of tokens per workgroup
+    blocks = grid_blocks((a.n_tokens + gather_tile<G>() - 1) / gather_tile<G>(), kBlock,
+                         resident_blocks<&attnres_gather_kernel<G, CH, VEC, BF16OUT, RING, SL>>());
+  }
+  hipLaunchKernelGGL((attnres_gather_kernel<G, CH, VEC, BF16OUT, RING, SL>), dim3(static_cast<unsigned>(blocks)),
                      dim3(kBlock), 0, stream, a);
 }
 
@@ -2703,11 +2793,13 @@ void launch_gather_ring(const GatherArgs& a, hipStream_t stream) {
 // 157.7 -> 165.9.
 template <int G, int CH, bool VEC, bool BF16OUT>
 void launch_gather(const GatherArgs& a, hipStream_t stream) {
-  constexpr int T = CH >= 4 ? 1 : 4 / CH;
-  if (a.n_reads >= 16 && few_waves((a.n_tokens + T - 1) / T, G)) {
-    launch_gather_ring<G, CH, VEC, BF16OUT, 3>(a, stream);
+  constexpr int T = gather_tokens<G, CH, 1>();
+  if (a.n_slots > 1) {
+    launch_gather_ring<G, CH, VEC, BF16OUT, 2, kGatherSlots>(a, stream);
+  } else if (a.n_reads >= 16 && few_waves((a.n_tokens + T - 1) / T, G)) {
+    launch_gather_ring<G, CH, VEC, BF16OUT, 3, 1>(a, stream);
   } else {
-    launch_gather_ring<G, CH, VEC, BF16OUT, 2>(a, stream);
+    launch_gather_ring<G, CH, VEC, BF16OUT, 2, 1>(a, stream);
   }
 }
 

@@ -92,6 +92,8 @@ enum attnres_status {
 #define ATTNRES_DTYPE_BF16 1
 /* Reads one attnres_hip_bank_gather launch takes (more take further launches). */
 #define ATTNRES_MAX_GATHER_READS 48
+/* Slots one attnres_hip_bank_gather_slots launch forms. */
+#define ATTNRES_GATHER_SLOTS 4
 
 /* Library version string; the Python package's __version__ (e.g. "2.0.1+mi355x.1"). */
 const char* attnres_hip_version(void);
@@ -386,6 +388,26 @@ int attnres_hip_bank_gather(const void* values, int64_t row_stride, int64_t n_to
                             int64_t width, const attnres_gather_read* reads,
                             int64_t n_reads, void* grad, int grad_dtype, int accumulate,
                             void* stream);
+
+/*
+ * The same for a slot whose sums are partly formed already, or for several
+ * slots at once:
+ *   - n_slots = 1: grad = base + the reads' sums (base: contiguous FP32 [N, D];
+ *     NULL: none), stored once as grad_dtype;
+ *   - n_slots = ATTNRES_GATHER_SLOTS: also the FP32 sums of the slots at the
+ *     reads' positions - 1, - 2, ..., written to partial[n_slots - 1, N, D]
+ *     (contiguous FP32).  Their rows lie slot_stride, 2 * slot_stride, ...
+ *     elements before `values`; every read's position is at least n_slots - 1.
+ *     The dO rows, which all the slots share, are read once instead of once
+ *     per slot.
+ * One launch: at most ATTNRES_MAX_GATHER_READS reads, all of one rank (else
+ * ATTNRES_ERR_SHAPE).  No counterpart in the reference; used by
+ * attnres.SourceBank.
+ */
+int attnres_hip_bank_gather_slots(const void* values, int64_t row_stride, int64_t slot_stride, int64_t n_slots,
+                                  int64_t n_tokens, int64_t width, const attnres_gather_read* reads,
+                                  int64_t n_reads, const float* base, void* grad, int grad_dtype, float* partial,
+                                  void* stream);
 
 /*
  * Block-schedule partial sum: out[i] = prev[i] + emitted[i] (FP32 arithmetic,
