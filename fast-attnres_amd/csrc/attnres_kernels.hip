@@ -13,7 +13,9 @@
 // lane owns CH chunks of 8 consecutive BF16 elements (one 16-byte load), the
 // chunks of a row interleaved across the group so that one load instruction
 // of a wavefront reads a contiguous span:
-//     element d of chunk c, lane l:  d = (c*G + l)*8 + e,  e in [0, 8).
+//     element d of chunk c, lane l:  d = (c*G + l)*8 + e,  e in [0, 8)
+// (the last chunk of a row whose width is no multiple of 8 is moved back; see
+// chunk_pos).
 // G is 16/32/64 (one or several tokens per wavefront; sums over the group are
 // DPP butterflies inside 16-lane rows plus lane reads across rows) or 256
 // (one token per workgroup for D > 4096; the four wave sums meet in LDS).
@@ -23,7 +25,9 @@
 // packed BF16 words feed v_dot2_f32_bf16 for the key sum of squares and the
 // query dot; the online softmax (running max, running sum, FP32 accumulator
 // of the full row) is updated; the per-source logit and 1/rms and the
-// per-token (max, 1/sum) are saved for the backward.
+// per-token (max, 1/sum) are saved for the backward.  Token blocks of one, two
+// or four tokens (attnres_fwd_block_kernel) and, for few tokens, a workgroup per
+// token (attnres_fwd_few_kernel) form the same sums; see launch_fwd.
 //
 // Backward.  A grid of up to two resident grids; group g takes tokens g,
 // g + groups, ... so that the groups work on neighbouring tokens at any time
@@ -274,7 +278,9 @@ __device__ __forceinline__ void store_refine(int8_t* __restrict__ refine, int d0
     } else {
       const int own = D & (kVec - 1);  // uniform
       if (own & 4) *reinterpret_cast<u32_at1*>(refine + D - 4) = r.y;
-      if (own & 2) *reinterpret_cast<u16_at1*>(refine + D - (own & 4) - 2) = static_cast<uint16_t>(((own & 4) ? r.x : r.y) >> 16);
+      if (own & 2) {
+        *reinterpret_cast<u16_at1*>(refine + D - (own & 4) - 2) = static_cast<uint16_t>(((own & 4) ? r.x : r.y) >> 16);
+      }
       if (own & 1) {  // byte 8 - own of the chunk: the odd byte of its pair
         const uint32_t word = (own & 4) ? r.x : r.y;
         refine[D - own] = static_cast<int8_t>((own & 2) ? (word >> 8) : (word >> 24));
@@ -670,17 +676,11 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_kernel(const FwdArgs<Rows>
 // span) rather than several sources of one token, rows a power-of-two source
 // stride apart that can fall into the same DRAM banks.  Per-token arithmetic
 // is the one-token kernel's (same sums in the same order): bit-identical
-// results.  Used at D = R = 2048 with T = 2, NBT = 2 (four rows in flight,
-// two per token, 206 VGPRs, two waves per SIMD) for 5 <= S <= 12, and with
-// T = 4, NBT = 1 (one row per token, 259 registers, one wave per SIMD) for
-// S >= 24; with T = 2, NBT = 1 for 64 lanes of 8 chunks (2048 < D <= 4096,
-// masked or not) from S = 13, for shorter rows of 64 lanes of 4 chunks
-// (1024 < D < 2048) and for workgroup-wide groups (4096 < D <= 8192) from
-// S = 5; with 32-lane groups (two per wavefront) for 128 < D <= 512 (T = 2,
-// NBT = 2) from S = 5 and for 512 < D < 1024 (T = 2, NBT = 1) from S = 9; see
-// launch_fwd for the measurements.  T = 4 forced to two waves
-// per SIMD (256 VGPRs) took 317-349 against 299-323 us at c2; the query words
-// read from LDS instead of registers made no difference.
+// results.  T = 1 is one token per group with NBT rows in flight and the output
+// formed once after the loop, for grids too small to hide latency otherwise.
+// launch_fwd states which shape serves which read and what each measured.
+// T = 4 forced to two waves per SIMD (256 VGPRs) took 317-349 against 299-323 us
+// at c2; the query words read from LDS instead of registers made no difference.
 // Like the token-block backward, its timing is sensitive to code generation:
 // changes are measured before they are kept.
 template <int G, int CH, int T, int NBT, bool NOMASK, bool VEC, class Rows>
@@ -2321,7 +2321,7 @@ inline int64_t device_cus() {
 // S=25, N=16384, D=2048: 645 -> 637; S=9, N=8192, D=8192: 492 -> 483;
 // S=25, N=2048, D=1024: 54 -> 47 (R=D), 55 -> 48 (R=256); but at N=16384,
 // D=1024 two rows are 0.8% slower (occupancy 2 either way), and the
-// accumulating and element-wise variants spill with two.  Rows of 8 chunks
+// accumulating variants spill with two.  Rows of 8 chunks
 // (64 lanes, D <= 4096) keep two rows without spilling only unmasked, and
 // are 2-3% slower with them (S=25, N=16384, D=R=4096: 1273 -> 1316; with the
 // iterative-minreg scheduler of the (64, 8) backward unit too: S=25 1295.5 ->
@@ -2387,7 +2387,7 @@ void launch_fwd_block(const FwdArgs<Rows>& a, hipStream_t stream) {
 // streaming kernels still hide their latency; wider rows move enough bytes per
 // token to get there sooner.  Measured on MI355X (no-grad forwards in a
 // replayed graph, us per read, streaming -> this): one token, S = 25: D = 2048:
-// 44.0 -> 7.3, D = 1024: 17.4 -> 5.4, D = 4096: 36.3 -> 10.9; S = 2, D = 1024:
+// 44.0 -> 7.3, D = 1024: 17.4 -> 5.4, D = 4096: 36.3 -> 9.2; S = 2, D = 1024:
 // 4.4 -> 3.7; 16 tokens, S = 48, D = 1024: 32.0 -> 8.0; 256 tokens: S = 25,
 // D = 2048: 56.9 -> 11.8, S = 9, D = 8192: 21.7 -> 18.0, S = 25, D = 256: 19.2
 // -> 7.8; 512 tokens: S = 25, D = 1024: 19.5 -> 13.7, S = 48, D = 2048: 35.4 ->
@@ -2474,7 +2474,10 @@ inline FwdBlockShape fwd_block_shape(int G, int CH, bool whole, bool nomask, int
     return S < 9 ? FwdBlockShape{0, 0} : whole ? FwdBlockShape{2, 2} : FwdBlockShape{2, 1};
   }
   if (CH == 8) return S > kPersistentFwdMaxSources ? FwdBlockShape{2, 1} : FwdBlockShape{0, 0};
-  if (CH == 4 && G == 64 && whole) return !nomask ? FwdBlockShape{1, 4} : S <= 12 ? FwdBlockShape{2, 2} : S < 24 ? FwdBlockShape{1, 4} : FwdBlockShape{4, 1};
+  if (CH == 4 && G == 64 && whole) {
+    if (!nomask) return {1, 4};
+    return S <= 12 ? FwdBlockShape{2, 2} : S < 24 ? FwdBlockShape{1, 4} : FwdBlockShape{4, 1};
+  }
   if (CH > 4 || (G == kBlock && CH == 3)) return S < 9 ? FwdBlockShape{0, 0} : FwdBlockShape{4, 1};
   return {2, 1};
 }
@@ -2808,7 +2811,10 @@ void launch_gather(const GatherArgs& a, hipStream_t stream) {
 // 64 lanes x 4 chunks took 204 VGPRs, 256 x 1 far fewer).
 template <int G, int CH>
 void launch_gather_geometry(const GatherArgs& a, bool vec, hipStream_t stream) {
-  constexpr int kLanes = G * CH > kBlock / 2 ? kBlock : G * CH > kBlock / 4 ? kBlock / 2 : G * CH > kBlock / 8 ? kBlock / 4 : G * CH;
+  constexpr int kLanes = G * CH > kBlock / 2   ? kBlock  // the power of two that holds the row's chunks
+                         : G * CH > kBlock / 4 ? kBlock / 2
+                         : G * CH > kBlock / 8 ? kBlock / 4
+                                               : G * CH;
   constexpr int kChunks = (G * CH + kLanes - 1) / kLanes;
   if (vec) {
     if (a.bf16_out) launch_gather<kLanes, kChunks, true, true>(a, stream);
