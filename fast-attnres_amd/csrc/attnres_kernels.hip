@@ -545,8 +545,6 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_kernel(const FwdArgs<Rows>
     }
   }
 
-  // acc needs no reset between tokens: with run_max = -inf the first
-  // source of a token rescales the old (finite) contents by exp(-inf) = 0.
   float acc[CH][kVec];
 #pragma unroll
   for (int c = 0; c < CH; ++c)
@@ -630,7 +628,6 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_kernel(const FwdArgs<Rows>
     }
 
     if (s == S - 1) {  // token complete: normalise and store the output row
-      // Normalised in place: the next token's first source rescales acc by 0.
       const float inv_sum = 1.0f / run_sum;
 #pragma unroll
       for (int c = 0; c < CH; ++c)
@@ -647,6 +644,12 @@ __global__ void __launch_bounds__(kBlock) attnres_fwd_kernel(const FwdArgs<Rows>
         a.stats[token] = run_max;
         a.stats[a.n_tokens + token] = inv_sum;
       }
+      // The next token starts from zero: rescaling by exp(-inf) = 0 would hand it
+      // a NaN or an infinity of this one.
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int e = 0; e < kVec; ++e) acc[c][e] = 0.0f;
       run_max = -INFINITY;
       run_sum = 0.0f;
     }
