@@ -581,6 +581,8 @@ struct BankPushSum : public torch::autograd::Function<BankPushSum> {
     Tensor grad = bank->take(ctx->saved_data["slot"].toInt(), dtype);
     if (grad.defined()) grad = grad.to(dtype);
     if (grads[0].defined()) grad = grad.defined() ? grads[0] + grad : grads[0];
+    // neither the partial nor the slot was used: a zero gradient, not an absent one
+    if (!grad.defined()) grad = torch::zeros(bank->values.sizes().slice(1), bank->values.options().dtype(dtype));
     const bool token = ctx->saved_data["token"].toBool();
     return {Tensor(), Tensor(), grad, grad, token ? torch::empty({0}, bank->values.options().dtype(dtype)) : Tensor()};
   }
@@ -588,7 +590,8 @@ struct BankPushSum : public torch::autograd::Function<BankPushSum> {
 
 // A read of the bank's slots.  Always saves the refinement (its backward
 // kernels read it); the backward leaves dv to the slots' gathers, or adds it
-// to their FP32 sums.
+// to their FP32 sums.  A read whose output received no gradient counts as one
+// with a zero gradient: its query and sources get zeros, not nothing.
 struct BankRead : public torch::autograd::Function<BankRead> {
   static Tensor forward(AutogradContext* ctx, const c10::intrusive_ptr<BankState>& bank, int64_t count, int64_t tail,
                         const Tensor& query, double eps, double scale, const Tensor& token) {
@@ -611,7 +614,6 @@ struct BankRead : public torch::autograd::Function<BankRead> {
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     variable_list result(7);  // bank, count, tail, query, eps, scale, token
-    if (!grads[0].defined()) return result;
     const auto bank = bank_of(ctx);
     const Slots slots{ctx->saved_data["count"].toInt(), ctx->saved_data["tail"].toInt()};
     const float scale = static_cast<float>(ctx->saved_data["scale"].toDouble());
@@ -620,7 +622,8 @@ struct BankRead : public torch::autograd::Function<BankRead> {
     const Tensor& like = bank->values;
     const int64_t S = slots.size(), N = bank->tokens, D = bank->width, R = query.numel();
     const c10::DeviceGuard guard(like.device());
-    const Tensor grad_out = grads[0].to(torch::kBFloat16).contiguous();
+    const Tensor grad_out = grads[0].defined() ? grads[0].to(torch::kBFloat16).contiguous()
+                                               : torch::zeros(like.sizes().slice(1), like.options());
     const StatePointers state = pool_pointers(pool, pool_layout(N, S, D, true), true);
     Tensor grad_query = bf16_empty({R}, like);
     Tensor workspace = dq_workspace(N, D, R, like);
