@@ -379,11 +379,19 @@ struct BankState : public torch::CustomClassHolder {
   std::vector<char> written;
   std::vector<std::vector<Pending>> pending;
   std::vector<Tensor> partial;  // FP32 sums of a slot's earlier reads (gather_block)
-  std::vector<char> wanted;     // the slot's source requires a gradient
+
+  // A slot's push node, whose first `inputs` edges lead to the slot's source (or
+  // to the terms of its sum); empty when the push recorded none.  Weak: the node
+  // holds this state.
+  struct PushNode {
+    std::weak_ptr<torch::autograd::Node> node;
+    size_t inputs = 0;
+  };
+  std::vector<PushNode> push_nodes;
 
   BankState(int64_t capacity_, bool gather_, bool bf16_gather_, const Tensor& source)
       : capacity(capacity_), gather(gather_), bf16_gather(bf16_gather_), written(capacity_, 0), pending(capacity_),
-        partial(capacity_), wanted(capacity_, 0) {
+        partial(capacity_), push_nodes(capacity_) {
     std::vector<int64_t> shape{capacity};
     shape.insert(shape.end(), source.sizes().begin(), source.sizes().end());
     values = bf16_empty(shape, source);
@@ -406,17 +414,35 @@ struct BankState : public torch::CustomClassHolder {
     pass = current;
   }
 
+  // Called by a Python thread, which lets go of its lock first: a backward call
+  // may hold `mutex` and need that lock to free a tensor.
+  void set_push_node(int64_t slot, const Tensor& token, size_t inputs) {
+    const py::gil_scoped_release release;
+    const std::lock_guard<std::mutex> lock(mutex);
+    push_nodes[slot] = {token.grad_fn(), inputs};
+  }
+
+  // Whether the running backward pass computes a gradient for the slot's source.
+  bool wanted(int64_t slot) const {
+    const auto node = push_nodes[slot].node.lock();
+    if (!node) return false;
+    for (size_t i = 0; i < push_nodes[slot].inputs; ++i) {
+      if (node->task_should_compute_output(i)) return true;
+    }
+    return false;
+  }
+
   // A slot with many reads also forms the FP32 sums of the slots before it
   // over the same reads, whose dO rows are then read once for all of them; the
   // slots add what reads they get later to those sums.  Only where the reads
-  // saw these slots one position apart (a Full schedule's prefixes) and their
-  // sources want gradients.  A block writes and reads 8 bytes of sums per
+  // saw these slots one position apart (a Full schedule's prefixes) and the pass
+  // computes their sources' gradients, so every sum is taken in this pass.  A block writes and reads 8 bytes of sums per
   // element and slot to save 2 per read, so it pays from about 9 reads on.
   bool gather_block(int64_t slot, const std::vector<Pending>& reads) const {
     if (reads.size() < kBlockReads || slot < ATTNRES_GATHER_SLOTS - 1) return false;
     for (int64_t k = 1; k < ATTNRES_GATHER_SLOTS; ++k) {
       const std::vector<Pending>& lower = pending[slot - k];
-      if (!wanted[slot - k] || partial[slot - k].defined() || lower.size() != reads.size()) return false;
+      if (!wanted(slot - k) || partial[slot - k].defined() || lower.size() != reads.size()) return false;
       for (size_t i = 0; i < reads.size(); ++i) {
         if (lower[i].record != reads[i].record || lower[i].position != reads[i].position - k) return false;
       }
@@ -440,7 +466,7 @@ struct BankState : public torch::CustomClassHolder {
     reads.swap(pending[slot]);
     Tensor base;
     std::swap(base, partial[slot]);
-    if (reads.empty() || !wanted[slot]) return base;
+    if (reads.empty() || !wanted(slot)) return base;
     std::vector<attnres_gather_read> table;
     table.reserve(reads.size());
     bool one_launch = reads.size() <= ATTNRES_MAX_GATHER_READS;
@@ -534,7 +560,6 @@ struct BankPush : public torch::autograd::Function<BankPush> {
                         const Tensor& source, const std::optional<Tensor>& previous) {
     const c10::DeviceGuard guard(source.device());
     bank->values.select(0, slot).copy_(source);
-    bank->wanted[slot] = source.requires_grad() ? 1 : 0;
     ctx->set_materialize_grads(false);
     ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
     ctx->saved_data["slot"] = slot;
@@ -566,7 +591,6 @@ struct BankPushSum : public torch::autograd::Function<BankPushSum> {
                                   b.scalar_type() == torch::kFloat32 ? ATTNRES_DTYPE_F32 : ATTNRES_DTYPE_BF16,
                                   b.numel(), partial.data_ptr(), bank->slot_rows(slot), current_stream(b)),
           "attnres partial sum");
-    bank->wanted[slot] = prev.requires_grad() || emitted.requires_grad() ? 1 : 0;
     ctx->set_materialize_grads(false);
     ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
     ctx->saved_data["slot"] = slot;
@@ -686,12 +710,15 @@ struct BankRead : public torch::autograd::Function<BankRead> {
 
 Tensor bank_push(const c10::intrusive_ptr<BankState>& bank, int64_t slot, const Tensor& source,
                  const std::optional<Tensor>& previous) {
-  return BankPush::apply(bank, slot, source, previous);
+  Tensor token = BankPush::apply(bank, slot, source, previous);
+  bank->set_push_node(slot, token, 1);
+  return token;
 }
 
 std::tuple<Tensor, Tensor> bank_push_sum(const c10::intrusive_ptr<BankState>& bank, int64_t slot, const Tensor& prev,
                                          const Tensor& emitted, const std::optional<Tensor>& previous) {
   const variable_list results = BankPushSum::apply(bank, slot, prev, emitted, previous);
+  bank->set_push_node(slot, results[1], 2);
   return {results[0], results[1]};
 }
 

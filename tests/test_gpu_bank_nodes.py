@@ -68,3 +68,42 @@ def test_a_read_without_an_upstream_gradient_gives_zero_gradients(gradients):
     expected = torch.autograd.grad(second.float().sum(), [source, later, query2])
     for a, b in zip((grads[0], grads[1], grads[3]), expected):
         assert torch.equal(a, b)
+
+
+def _full_schedule(sources, queries, gradients="gather", ungraded=()):
+    """Push a source, read all so far, over and over; sources whose index is in
+    ``ungraded`` are pushed with grad mode off."""
+    bank = SourceBank(len(sources), gradients=gradients)
+    outs = []
+    for i, (source, query) in enumerate(zip(sources, queries)):
+        with torch.set_grad_enabled(i not in ungraded):
+            bank.push(source)
+        outs.append(bank.read(query))
+    return outs
+
+
+def _kept(outs, inputs, grads):
+    """The gradients of one pass and the bytes that it leaves allocated besides them."""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    results = torch.autograd.grad(outs, inputs, grads, retain_graph=True)
+    torch.cuda.synchronize()
+    return results, torch.cuda.memory_allocated() - before - sum(r.numel() * r.element_size() for r in results)
+
+
+# 16 reads: slot 7 is the last one with nine of them, the first that may form the sums of slots 6, 5 and 4 too
+@pytest.mark.parametrize("ungraded", [(), (0, 1, 2, 3, 4, 5, 6)])
+def test_a_pass_forms_no_sums_it_was_not_asked_for(ungraded):
+    torch.manual_seed(7)
+    tokens, width, reads = 512, 1024, 16
+    sources = [_source(tokens, width=width) for _ in range(reads)]
+    queries = [_query(width) for _ in range(reads)]
+    grads = [torch.randn(tokens, width, device="cuda", dtype=torch.bfloat16) for _ in range(reads)]
+    inputs = [sources[7]] if not ungraded else sources[7:]
+    results, kept = _kept(_full_schedule(sources, queries, ungraded=ungraded), inputs, grads)
+    # the reads' coefficients (12 bytes per source and token) may stay until the next pass; FP32 sums may not
+    assert kept < tokens * width * 4, f"{kept} bytes kept"
+    expected = torch.autograd.grad(_full_schedule(sources, queries, "accumulate", ungraded), inputs, grads)
+    for a, b in zip(results, expected):
+        # FP32 sums of 2 * reads terms in another order: 2^-24 of their magnitude each, as in the tests of blocks
+        torch.testing.assert_close(a, b, rtol=2.0**-18, atol=2.0**-18 * float(b.abs().max()))
