@@ -26,6 +26,7 @@
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 
 #include <torch/csrc/autograd/graph_task.h>
@@ -350,17 +351,35 @@ Tensor sources_read(const Tensor& query, double eps, double scale, const std::ve
 
 // ------------------------------------------------------------- source bank
 
+// The current stream of the tensor's device (as torch sees it: the stream an
+// allocation made now belongs to).
+c10::Stream stream_of(const Tensor& tensor) {
+  return c10::impl::VirtualGuardImpl(tensor.device().type()).getStream(tensor.device());
+}
+
+// `tensor`, known to the allocator as used on stream `made`, is used by kernels
+// of stream `now` (use_here: the current one): its memory is not handed out again before they end.
+void use_on(const c10::Stream& now, const Tensor& tensor, const c10::Stream& made) {
+  if (now != made) {
+    c10::impl::VirtualGuardImpl(now.device_type()).recordDataPtrOnStream(tensor.storage().data_ptr(), now);
+  }
+}
+void use_here(const Tensor& tensor, const c10::Stream& made) { use_on(stream_of(tensor), tensor, made); }
+
 // The slots of a SourceBank and one backward pass's gradient bookkeeping,
 // used by the nodes below (attnres/shared.py states the scheme).  The nodes
 // hold it and it holds no token, so nothing closes a cycle.  Backward nodes
 // run without Python's lock, possibly on several threads: `mutex` guards the
-// pass's bookkeeping.
+// pass's bookkeeping.  Pushes and reads may run on different streams: autograd
+// orders their backward kernels (by the tokens), and what one node allocates and
+// another uses is kept until that use ends (use_here).
 struct BankState : public torch::CustomClassHolder {
   // One read's gathered terms: its dO, the query on row positions and the
   // coefficients [3, count, N]; kept until the gathers of its slots are enqueued.
   struct Record {
     Tensor grad_out, query_row, coef;
     int64_t count, rank;
+    c10::Stream stream;  // of the read's backward
   };
   struct Pending {
     std::shared_ptr<Record> record;
@@ -371,14 +390,20 @@ struct BankState : public torch::CustomClassHolder {
   bool gather;       // gradients="gather", else accumulated FP32 sums
   bool bf16_gather;  // a BF16 source's gradient is stored as BF16 by its one gather launch
   Tensor values;     // [capacity, ..., D] BF16
+  c10::Stream values_stream;
   int64_t tokens = 0, width = 0;
 
   std::mutex mutex;
   int64_t pass = -1;
   Tensor sums;  // [capacity, ..., D] FP32 (accumulate)
+  std::optional<c10::Stream> sums_stream;
   std::vector<char> written;
   std::vector<std::vector<Pending>> pending;
-  std::vector<Tensor> partial;  // FP32 sums of a slot's earlier reads (gather_block)
+  struct Partial {  // FP32 sums of a slot's earlier reads (gather_block)
+    Tensor sum;
+    std::optional<c10::Stream> stream;
+  };
+  std::vector<Partial> partial;
 
   // A slot's push node, whose first `inputs` edges lead to the slot's source (or
   // to the terms of its sum); empty when the push recorded none.  Weak: the node
@@ -390,8 +415,8 @@ struct BankState : public torch::CustomClassHolder {
   std::vector<PushNode> push_nodes;
 
   BankState(int64_t capacity_, bool gather_, bool bf16_gather_, const Tensor& source)
-      : capacity(capacity_), gather(gather_), bf16_gather(bf16_gather_), written(capacity_, 0), pending(capacity_),
-        partial(capacity_), push_nodes(capacity_) {
+      : capacity(capacity_), gather(gather_), bf16_gather(bf16_gather_), values_stream(stream_of(source)),
+        written(capacity_, 0), pending(capacity_), partial(capacity_), push_nodes(capacity_) {
     std::vector<int64_t> shape{capacity};
     shape.insert(shape.end(), source.sizes().begin(), source.sizes().end());
     values = bf16_empty(shape, source);
@@ -410,7 +435,7 @@ struct BankState : public torch::CustomClassHolder {
     sums = Tensor();
     std::fill(written.begin(), written.end(), 0);
     for (auto& list : pending) list.clear();
-    for (Tensor& sum : partial) sum = Tensor();
+    for (Partial& lower : partial) lower = Partial();
     pass = current;
   }
 
@@ -442,7 +467,7 @@ struct BankState : public torch::CustomClassHolder {
     if (reads.size() < kBlockReads || slot < ATTNRES_GATHER_SLOTS - 1) return false;
     for (int64_t k = 1; k < ATTNRES_GATHER_SLOTS; ++k) {
       const std::vector<Pending>& lower = pending[slot - k];
-      if (!wanted(slot - k) || partial[slot - k].defined() || lower.size() != reads.size()) return false;
+      if (!wanted(slot - k) || partial[slot - k].sum.defined() || lower.size() != reads.size()) return false;
       for (size_t i = 0; i < reads.size(); ++i) {
         if (lower[i].record != reads[i].record || lower[i].position != reads[i].position - k) return false;
       }
@@ -460,19 +485,25 @@ struct BankState : public torch::CustomClassHolder {
     if (!gather) {
       if (!written[slot]) return Tensor();
       written[slot] = 0;
+      use_here(sums, *sums_stream);
       return sums.select(0, slot);
     }
     std::vector<Pending> reads;
     reads.swap(pending[slot]);
-    Tensor base;
-    std::swap(base, partial[slot]);
+    Partial earlier;
+    std::swap(earlier, partial[slot]);
+    const Tensor base = earlier.sum;
+    const c10::Stream now = stream_of(values);
+    if (base.defined()) use_on(now, base, *earlier.stream);
     if (reads.empty() || !wanted(slot)) return base;
+    use_on(now, values, values_stream);
     std::vector<attnres_gather_read> table;
     table.reserve(reads.size());
     bool one_launch = reads.size() <= ATTNRES_MAX_GATHER_READS;
     for (const Pending& p : reads) {
       const Record& r = *p.record;
       one_launch = one_launch && r.rank == reads[0].record->rank;
+      for (const Tensor* term : {&r.grad_out, &r.query_row, &r.coef}) use_on(now, *term, r.stream);
       table.push_back({r.grad_out.data_ptr(), r.query_row.data_ptr(), r.coef.data_ptr<float>(), r.count, p.position,
                        r.rank});
     }
@@ -504,7 +535,7 @@ struct BankState : public torch::CustomClassHolder {
           "attnres source-bank gather");
     if (block) {
       for (int64_t k = 1; k < ATTNRES_GATHER_SLOTS; ++k) {
-        partial[slot - k] = lower.select(0, k - 1);
+        partial[slot - k] = {lower.select(0, k - 1), now};
         pending[slot - k].clear();
       }
     }
@@ -532,6 +563,7 @@ struct SlotTable {
 void bank_forward(const BankState& bank, const Slots& slots, const Tensor& query, double eps, double scale,
                   const Tensor& out, const StatePointers& state) {
   const int64_t S = slots.size(), N = bank.tokens, D = bank.width, R = query.numel();
+  use_here(bank.values, bank.values_stream);
   if (slots.prefix()) {
     check(attnres_hip_packed_forward(bank.values.data_ptr(), N * D, D, S, N, D, query.data_ptr(), R,
                                      static_cast<float>(eps), static_cast<float>(scale), out.data_ptr(), state.refine,
@@ -559,6 +591,7 @@ struct BankPush : public torch::autograd::Function<BankPush> {
   static Tensor forward(AutogradContext* ctx, const c10::intrusive_ptr<BankState>& bank, int64_t slot,
                         const Tensor& source, const std::optional<Tensor>& previous) {
     const c10::DeviceGuard guard(source.device());
+    use_here(bank->values, bank->values_stream);
     bank->values.select(0, slot).copy_(source);
     ctx->set_materialize_grads(false);
     ctx->saved_data["bank"] = c10::IValue::make_capsule(bank);
@@ -587,6 +620,7 @@ struct BankPushSum : public torch::autograd::Function<BankPushSum> {
     const c10::DeviceGuard guard(emitted.device());
     const Tensor a = prev.contiguous(), b = emitted.contiguous();
     Tensor partial = torch::empty(b.sizes(), b.options());
+    use_here(bank->values, bank->values_stream);
     check(attnres_hip_partial_sum(a.data_ptr(), b.data_ptr(),
                                   b.scalar_type() == torch::kFloat32 ? ATTNRES_DTYPE_F32 : ATTNRES_DTYPE_BF16,
                                   b.numel(), partial.data_ptr(), bank->slot_rows(slot), current_stream(b)),
@@ -652,6 +686,7 @@ struct BankRead : public torch::autograd::Function<BankRead> {
     Tensor grad_query = bf16_empty({R}, like);
     Tensor workspace = dq_workspace(N, D, R, like);
     const auto stream = current_stream(like);
+    use_here(like, bank->values_stream);
     const std::lock_guard<std::mutex> lock(bank->mutex);
     bank->begin_pass();
     if (bank->gather) {
@@ -677,10 +712,15 @@ struct BankRead : public torch::autograd::Function<BankRead> {
         query_row = torch::zeros({D}, query.options());
         query_row.narrow(0, D - R, R).copy_(query);
       }
-      const auto record = std::make_shared<BankState::Record>(BankState::Record{grad_out, query_row, coef, S, R});
+      const auto record = std::make_shared<BankState::Record>(
+          BankState::Record{grad_out, query_row, coef, S, R, stream_of(like)});
       for (int64_t i = 0; i < S; ++i) bank->pending[slots.at(i)].push_back({record, i});
     } else {
-      if (!bank->sums.defined()) bank->sums = torch::empty(like.sizes(), like.options().dtype(torch::kFloat32));
+      if (!bank->sums.defined()) {
+        bank->sums = torch::empty(like.sizes(), like.options().dtype(torch::kFloat32));
+        bank->sums_stream = stream_of(like);
+      }
+      use_here(bank->sums, *bank->sums_stream);
       std::vector<uint8_t> flags;
       for (int64_t i = 0; i < S; ++i) flags.push_back(bank->written[slots.at(i)] ? 1 : 0);
       float* sums = bank->sums.data_ptr<float>();

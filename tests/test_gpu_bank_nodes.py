@@ -4,6 +4,7 @@ the nodes keep from one backward call to the next."""
 from __future__ import annotations
 
 import math
+import threading
 
 import pytest
 import torch
@@ -107,3 +108,80 @@ def test_a_pass_forms_no_sums_it_was_not_asked_for(ungraded):
     for a, b in zip(results, expected):
         # FP32 sums of 2 * reads terms in another order: 2^-24 of their magnitude each, as in the tests of blocks
         torch.testing.assert_close(a, b, rtol=2.0**-18, atol=2.0**-18 * float(b.abs().max()))
+
+
+class _Streams:
+    """Runs pieces of a program on chosen streams, each after all pieces before it."""
+
+    def __init__(self, *streams):
+        self.all = (torch.cuda.current_stream(), *streams)
+
+    def run(self, stream, piece):
+        for other in self.all:
+            if other is not stream:
+                stream.wait_stream(other)
+        with torch.cuda.stream(stream):
+            return piece()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("gradients", ["gather", "accumulate"])
+def test_pushes_and_reads_on_several_streams(gradients, dtype):
+    """Slots 10 to 15 are pushed on one stream, slots 0 to 9 on another and all
+    reads run on a third.  In the backward pass the gathers of slots 0 to 9 wait
+    behind other work of their stream, long after the pass has let go of the
+    reads' terms (third stream) and of the sums that slot 7's and later gathers
+    left for the slots before them; what the first and third stream allocate and
+    overwrite meanwhile must not reach those gathers."""
+    torch.manual_seed(8)
+    tokens, width, reads, cut = 4096, 256, 16, 10
+    sources = [_source(tokens, dtype=dtype, width=width) for _ in range(reads)]
+    queries = [_query(width) for _ in range(reads)]
+    grads = [torch.randn(tokens, width, device="cuda", dtype=torch.bfloat16) for _ in range(reads)]
+    inputs = (*sources, *queries)
+    expected = torch.autograd.grad(_full_schedule(sources, queries, gradients), inputs, grads)
+
+    high, low, reader = (torch.cuda.Stream() for _ in range(3))
+    streams = _Streams(high, low, reader)
+    bank = SourceBank(reads, gradients=gradients)
+    outs = []
+    for i, (source, query) in enumerate(zip(sources, queries)):
+        streams.run(low if i < cut else high, lambda: bank.push(source))
+        outs.append(streams.run(reader, lambda: bank.read(query)))
+    busy = torch.randn(8192, 8192, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(low):  # tens of milliseconds before the low slots' gathers
+        for _ in range(5):
+            product = busy @ busy
+    results = torch.autograd.grad(outs, inputs, grads)
+    rubbish = []
+    for stream in (reader, high):
+        with torch.cuda.stream(stream):
+            for count in range(1, reads + 1):
+                rubbish += [torch.empty(3, count, tokens, device="cuda").fill_(float("nan")) for _ in range(2)]
+            rubbish += [torch.empty(3, tokens, width, device="cuda").fill_(float("nan")) for _ in range(4)]
+            rubbish += [torch.empty(reads, tokens, width, device="cuda").fill_(float("nan")) for _ in range(2)]
+    torch.cuda.synchronize()
+    del product
+    for i, (a, b) in enumerate(zip(results, expected)):
+        assert torch.equal(a, b), f"gradient {i}"
+
+
+@pytest.mark.parametrize("gradients", ["gather", "accumulate"])
+def test_nodes_with_saved_tensor_hooks_and_on_another_thread(gradients):
+    torch.manual_seed(9)
+    sources = [_source(33) for _ in range(12)]
+    queries = [_query() for _ in range(12)]
+    grads = [torch.randn(33, _WIDTH, device="cuda", dtype=torch.bfloat16) for _ in range(12)]
+    inputs = (*sources, *queries)
+    expected = torch.autograd.grad(_full_schedule(sources, queries, gradients), inputs, grads)
+    with torch.autograd.graph.save_on_cpu():
+        outs = _full_schedule(sources, queries, gradients)
+    hooked = torch.autograd.grad(outs, inputs, grads)
+    outs = _full_schedule(sources, queries, gradients)
+    results = []
+    thread = threading.Thread(target=lambda: results.extend(torch.autograd.grad(outs, inputs, grads)))
+    thread.start()
+    thread.join()
+    for a, b, c in zip(hooked, results, expected):
+        assert torch.equal(a, c) and torch.equal(b, c)
