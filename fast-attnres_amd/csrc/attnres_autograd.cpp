@@ -495,7 +495,10 @@ struct BankState : public torch::CustomClassHolder {
     const Tensor base = earlier.sum;
     const c10::Stream now = stream_of(values);
     if (base.defined()) use_on(now, base, *earlier.stream);
-    if (reads.empty() || !wanted(slot)) return base;
+    if (!wanted(slot)) return Tensor();
+    // the sums of a block's slots lie in one allocation: an FP32 source receives a copy of its own
+    const auto own = [&] { return base.defined() && dtype == torch::kFloat32 ? base.clone() : base; };
+    if (reads.empty()) return own();
     use_on(now, values, values_stream);
     std::vector<attnres_gather_read> table;
     table.reserve(reads.size());
@@ -514,7 +517,7 @@ struct BankState : public torch::CustomClassHolder {
     const auto fp32 = values.options().dtype(torch::kFloat32);
     if (!one_launch) {
       const bool add = base.defined();
-      Tensor grad = add ? base : torch::empty(values.sizes().slice(1), fp32);
+      Tensor grad = add ? own() : torch::empty(values.sizes().slice(1), fp32);
       check(attnres_hip_bank_gather(slot_rows(slot), width, tokens, width, table.data(), count, grad.data_ptr(),
                                     grad_dtype, add ? 1 : 0, current_stream(values)),
             "attnres source-bank gather");

@@ -71,6 +71,14 @@ def test_a_read_without_an_upstream_gradient_gives_zero_gradients(gradients):
         assert torch.equal(a, b)
 
 
+def _close(actual, expected):
+    """FP32 sums of at most 64 terms in another order (2^-24 of their magnitude each, taken as 2^-18 of the
+    largest element), rounded to BF16 for BF16 sources: one unit in the last place, 2^-7 of the element."""
+    rtol = 2.0**-7 if expected.dtype == torch.bfloat16 else 2.0**-18
+    torch.testing.assert_close(actual.float(), expected.float(), rtol=rtol,
+                               atol=2.0**-18 * float(expected.float().abs().max()))
+
+
 def _full_schedule(sources, queries, gradients="gather", ungraded=()):
     """Push a source, read all so far, over and over; sources whose index is in
     ``ungraded`` are pushed with grad mode off."""
@@ -106,8 +114,7 @@ def test_a_pass_forms_no_sums_it_was_not_asked_for(ungraded):
     assert kept < tokens * width * 4, f"{kept} bytes kept"
     expected = torch.autograd.grad(_full_schedule(sources, queries, "accumulate", ungraded), inputs, grads)
     for a, b in zip(results, expected):
-        # FP32 sums of 2 * reads terms in another order: 2^-24 of their magnitude each, as in the tests of blocks
-        torch.testing.assert_close(a, b, rtol=2.0**-18, atol=2.0**-18 * float(b.abs().max()))
+        _close(a, b)
 
 
 class _Streams:
@@ -185,3 +192,33 @@ def test_nodes_with_saved_tensor_hooks_and_on_another_thread(gradients):
     thread.join()
     for a, b, c in zip(hooked, results, expected):
         assert torch.equal(a, c) and torch.equal(b, c)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("case", ["push-all-then-read", "early-reads-of-other-ranks"])
+def test_sums_left_for_lower_slots_are_each_slots_own(case, dtype):
+    """Slots that get no read after a block formed their sums, and slots whose
+    later reads need several launches (two ranks), take the sums as they are or
+    add to them; every gradient has memory of its own."""
+    torch.manual_seed(10)
+    count, tokens = 16, 40
+    sources = [_source(tokens, dtype=dtype) for _ in range(count)]
+    # slot 7 is the first with nine reads; slots 5 and 4 then get reads 6 and 5 (and 4), of two ranks
+    ranks = [_WIDTH // 2 if case.startswith("early") and i in (4, 6) else _WIDTH for i in range(count)]
+    queries = [_query(rank) for rank in ranks]
+    grads = [torch.randn(tokens, _WIDTH, device="cuda", dtype=torch.bfloat16) for _ in range(count)]
+
+    def outputs(gradients):
+        if case.startswith("early"):
+            return _full_schedule(sources, queries, gradients)
+        bank = SourceBank(count, gradients=gradients)
+        for source in sources:
+            bank.push(source)
+        return [bank.read(query) for query in queries]
+
+    results = torch.autograd.grad(outputs("gather"), sources, grads)
+    for a, b in zip(results, torch.autograd.grad(outputs("accumulate"), sources, grads)):
+        held, needed = a.untyped_storage().nbytes(), a.numel() * a.element_size()
+        assert held == needed
+        _close(a, b)
+    assert len({a.untyped_storage().data_ptr() for a in results}) == count
