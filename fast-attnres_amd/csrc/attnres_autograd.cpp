@@ -26,6 +26,7 @@
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 
@@ -396,7 +397,7 @@ struct BankState : public torch::CustomClassHolder {
   std::mutex mutex;
   int64_t pass = -1;
   Tensor sums;  // [capacity, ..., D] FP32 (accumulate)
-  std::optional<c10::Stream> sums_stream;
+  std::optional<c10::Stream> sums_stream, sums_last;  // allocated on, last added to on
   std::vector<char> written;
   std::vector<std::vector<Pending>> pending;
   struct Partial {  // FP32 sums of a slot's earlier reads (gather_block)
@@ -437,6 +438,19 @@ struct BankState : public torch::CustomClassHolder {
     for (auto& list : pending) list.clear();
     for (Partial& lower : partial) lower = Partial();
     pass = current;
+  }
+
+  // The current stream adds to the sums next, after what other streams added (no
+  // autograd edge orders the backward kernels of two reads).
+  void add_to_sums_here() {
+    const c10::Stream now = stream_of(sums);
+    if (now != *sums_last) {
+      c10::Event added(now.device_type());
+      added.record(*sums_last);
+      added.block(now);
+      sums_last = now;
+    }
+    use_on(now, sums, *sums_stream);
   }
 
   // Called by a Python thread, which lets go of its lock first: a backward call
@@ -721,9 +735,9 @@ struct BankRead : public torch::autograd::Function<BankRead> {
     } else {
       if (!bank->sums.defined()) {
         bank->sums = torch::empty(like.sizes(), like.options().dtype(torch::kFloat32));
-        bank->sums_stream = stream_of(like);
+        bank->sums_stream = bank->sums_last = stream_of(like);
       }
-      use_here(bank->sums, *bank->sums_stream);
+      bank->add_to_sums_here();
       std::vector<uint8_t> flags;
       for (int64_t i = 0; i < S; ++i) flags.push_back(bank->written[slots.at(i)] ? 1 : 0);
       float* sums = bank->sums.data_ptr<float>();

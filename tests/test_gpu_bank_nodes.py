@@ -133,12 +133,14 @@ class _Streams:
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("gradients", ["gather", "accumulate"])
-def test_pushes_and_reads_on_several_streams(gradients, dtype):
-    """Slots 10 to 15 are pushed on one stream, slots 0 to 9 on another and all
-    reads run on a third.  In the backward pass the gathers of slots 0 to 9 wait
+@pytest.mark.parametrize("readers", [1, 2])
+def test_pushes_and_reads_on_several_streams(gradients, dtype, readers):
+    """Slots 10 to 15 are pushed on one stream, slots 0 to 9 on another and the
+    reads run on a third (or a third and a fourth in turn, whose backward kernels
+    only the accumulated sums tie together).  In the backward pass the gathers of slots 0 to 9 wait
     behind other work of their stream, long after the pass has let go of the
-    reads' terms (third stream) and of the sums that slot 7's and later gathers
-    left for the slots before them; what the first and third stream allocate and
+    reads' terms and of the sums that slot 7's and later gathers
+    left for the slots before them; what the other streams allocate and
     overwrite meanwhile must not reach those gathers."""
     torch.manual_seed(8)
     tokens, width, reads, cut = 4096, 256, 16, 10
@@ -148,13 +150,13 @@ def test_pushes_and_reads_on_several_streams(gradients, dtype):
     inputs = (*sources, *queries)
     expected = torch.autograd.grad(_full_schedule(sources, queries, gradients), inputs, grads)
 
-    high, low, reader = (torch.cuda.Stream() for _ in range(3))
-    streams = _Streams(high, low, reader)
+    high, low, *reading = (torch.cuda.Stream() for _ in range(2 + readers))
+    streams = _Streams(high, low, *reading)
     bank = SourceBank(reads, gradients=gradients)
     outs = []
     for i, (source, query) in enumerate(zip(sources, queries)):
         streams.run(low if i < cut else high, lambda: bank.push(source))
-        outs.append(streams.run(reader, lambda: bank.read(query)))
+        outs.append(streams.run(reading[i % readers], lambda: bank.read(query)))
     busy = torch.randn(8192, 8192, device="cuda")
     torch.cuda.synchronize()
     with torch.cuda.stream(low):  # tens of milliseconds before the low slots' gathers
@@ -162,7 +164,7 @@ def test_pushes_and_reads_on_several_streams(gradients, dtype):
             product = busy @ busy
     results = torch.autograd.grad(outs, inputs, grads)
     rubbish = []
-    for stream in (reader, high):
+    for stream in (high, *reading):
         with torch.cuda.stream(stream):
             for count in range(1, reads + 1):
                 rubbish += [torch.empty(3, count, tokens, device="cuda").fill_(float("nan")) for _ in range(2)]
