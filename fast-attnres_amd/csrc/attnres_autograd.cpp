@@ -765,18 +765,24 @@ struct BankRead : public torch::autograd::Function<BankRead> {
   }
 };
 
+// The token after a push: with grad mode off it is the one before, so that later
+// reads still order themselves after (and reach) the pushes that want gradients.
+Tensor next_token(const Tensor& token, const std::optional<Tensor>& previous) {
+  return !token.requires_grad() && previous && previous->requires_grad() ? *previous : token;
+}
+
 Tensor bank_push(const c10::intrusive_ptr<BankState>& bank, int64_t slot, const Tensor& source,
                  const std::optional<Tensor>& previous) {
   Tensor token = BankPush::apply(bank, slot, source, previous);
   bank->set_push_node(slot, token, 1);
-  return token;
+  return next_token(token, previous);
 }
 
 std::tuple<Tensor, Tensor> bank_push_sum(const c10::intrusive_ptr<BankState>& bank, int64_t slot, const Tensor& prev,
                                          const Tensor& emitted, const std::optional<Tensor>& previous) {
   const variable_list results = BankPushSum::apply(bank, slot, prev, emitted, previous);
   bank->set_push_node(slot, results[1], 2);
-  return {results[0], results[1]};
+  return {results[0], next_token(results[1], previous)};
 }
 
 // No gradient wanted (grad mode off, or neither the query nor the sources --

@@ -4,6 +4,7 @@ the nodes keep from one backward call to the next."""
 from __future__ import annotations
 
 import math
+import operator
 import threading
 
 import pytest
@@ -224,3 +225,31 @@ def test_sums_left_for_lower_slots_are_each_slots_own(case, dtype):
         assert held == needed
         _close(a, b)
     assert len({a.untyped_storage().data_ptr() for a in results}) == count
+
+
+@pytest.mark.parametrize("gradients", ["gather", "accumulate"])
+def test_a_push_with_grad_mode_off_keeps_the_other_sources_gradients(gradients):
+    """Slots 2 and 3 (a push and a sum) are filled with grad mode off: the same
+    gradients as with sources that require none."""
+    torch.manual_seed(11)
+    sources = [_source() for _ in range(6)]
+    queries = [_query() for _ in range(6)]
+
+    def outputs(detached):
+        bank = SourceBank(6, gradients=gradients)
+        outs = []
+        for i, (source, query) in enumerate(zip(sources, queries)):
+            frozen = source.detach() if detached and i in (2, 3) else source
+            with torch.set_grad_enabled(detached or i not in (2, 3)):
+                if i == 3:
+                    bank.push_sum(frozen, frozen)
+                else:
+                    bank.push(frozen)
+            outs.append(bank.read(query).float().sum())
+        return outs
+
+    for reads in ([3], range(6)):  # the read right after them, or all reads
+        wanted = [s for i, s in enumerate(sources) if i < 2 or i in reads and i > 3] + [queries[i] for i in reads]
+        results = torch.autograd.grad(operator.itemgetter(*reads)(outputs(False)), wanted)
+        for a, b in zip(results, torch.autograd.grad(operator.itemgetter(*reads)(outputs(True)), wanted)):
+            assert torch.equal(a, b)
