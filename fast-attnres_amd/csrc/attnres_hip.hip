@@ -733,10 +733,11 @@ namespace attnres_hip {
 namespace {
 
 // The arguments both gather entries share: checked reads, and whether rows,
-// gradients and reads are 16-byte aligned.
+// gradients and reads are 16-byte aligned.  `one_launch`: why the reads must
+// fit one launch (nullptr: they need not).
 int check_gather(const char* name, const void* values, int64_t row_stride, int64_t n_tokens, int64_t width,
-                 const attnres_gather_read* reads, int64_t n_reads, const void* grad, int grad_dtype, bool one_launch,
-                 int64_t n_slots, bool* vec) {
+                 const attnres_gather_read* reads, int64_t n_reads, const void* grad, int grad_dtype,
+                 const char* one_launch, int64_t n_slots, bool* vec) {
   int st = check_shape(1, n_tokens, width, 1);
   if (st) return st;
   if (!values || !reads || !grad) return fail(ATTNRES_ERR_NULL_POINTER, "null pointer argument to %s", name);
@@ -748,8 +749,7 @@ int check_gather(const char* name, const void* values, int64_t row_stride, int64
     bool one_rank = true;
     for (int64_t r = 1; r < n_reads; ++r) one_rank = one_rank && reads[r].rank == reads[0].rank;
     if (n_reads > ATTNRES_MAX_GATHER_READS || !one_rank)
-      return fail(ATTNRES_ERR_SHAPE,
-                  "a BF16 gradient is written by one launch: accumulate=0, at most %d reads, all of one rank",
+      return fail(ATTNRES_ERR_SHAPE, "%s: %s, at most %d reads, all of one rank", name, one_launch,
                   ATTNRES_MAX_GATHER_READS);
   }
   *vec = width % kVec == 0 && aligned16(values) && aligned16(grad) && (row_stride % kVec == 0 || n_tokens == 1);
@@ -806,15 +806,14 @@ extern "C" {
 int attnres_hip_bank_gather(const void* values, int64_t row_stride, int64_t n_tokens, int64_t width,
                             const attnres_gather_read* reads, int64_t n_reads, void* grad, int grad_dtype,
                             int accumulate, void* stream) {
+  static const char* const kName = "attnres_hip_bank_gather";
   const bool bf16_out = grad_dtype == ATTNRES_DTYPE_BF16;
   bool vec = false;
-  const int st = check_gather("attnres_hip_bank_gather", values, row_stride, n_tokens, width, reads, n_reads, grad,
-                              grad_dtype, bf16_out, 1, &vec);
+  static const char* const kOneLaunch = "a BF16 gradient is written by one launch: accumulate=0";
+  const int st = check_gather(kName, values, row_stride, n_tokens, width, reads, n_reads, grad, grad_dtype,
+                              bf16_out ? kOneLaunch : nullptr, 1, &vec);
   if (st) return st;
-  if (bf16_out && accumulate)
-    return fail(ATTNRES_ERR_SHAPE,
-                "a BF16 gradient is written by one launch: accumulate=0, at most %d reads, all of one rank",
-                ATTNRES_MAX_GATHER_READS);
+  if (bf16_out && accumulate) return fail(ATTNRES_ERR_SHAPE, "%s: %s", kName, kOneLaunch);
   // One launch per run of at most kMaxGatherReads reads with the same rank
   // (in the caller's order); every launch after the first adds to grad.
   for (int64_t first = 0; first < n_reads;) {
@@ -837,8 +836,8 @@ int attnres_hip_bank_gather_slots(const void* values, int64_t row_stride, int64_
   if (n_slots != 1 && n_slots != ATTNRES_GATHER_SLOTS)
     return fail(ATTNRES_ERR_SHAPE, "n_slots=%lld is neither 1 nor %d", (long long)n_slots, ATTNRES_GATHER_SLOTS);
   bool vec = false;
-  const int st = check_gather(kName, values, row_stride, n_tokens, width, reads, n_reads, grad, grad_dtype, true,
-                              n_slots, &vec);
+  const int st = check_gather(kName, values, row_stride, n_tokens, width, reads, n_reads, grad, grad_dtype,
+                              "one launch", n_slots, &vec);
   if (st) return st;
   if (n_slots > 1 && !partial) return fail(ATTNRES_ERR_NULL_POINTER, "null pointer argument to %s", kName);
   if (slot_stride < 0) return fail(ATTNRES_ERR_STRIDE, "negative slot stride");

@@ -18,6 +18,8 @@ def test_bank_gather_slots_checks_its_arguments():
     reads = (_GatherRead * 49)(*[(_FAKE, _FAKE, _FAKE, 9, 5, 16)] * 49)
     assert _call(lib, reads, 2, n_slots=2) == _native.ERR_SHAPE and b"n_slots" in lib.attnres_hip_last_error()
     assert _call(lib, reads, 49) == _native.ERR_SHAPE and b"at most 48 reads" in lib.attnres_hip_last_error()
+    # the entry has no accumulate argument, and FP32 gradients take one launch too
+    assert b"accumulate" not in lib.attnres_hip_last_error() and b"BF16" not in lib.attnres_hip_last_error()
     assert _call(lib, reads, 0) == _native.ERR_SHAPE
     assert _call(lib, reads, 2, partial=None) == _native.ERR_NULL_POINTER
     assert _call(lib, reads, 2, values=None) == _native.ERR_NULL_POINTER
