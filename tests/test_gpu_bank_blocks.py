@@ -43,14 +43,15 @@ def _close(actual, expected, dtype):
     torch.testing.assert_close(actual.float(), expected.float(), rtol=rtol, atol=atol)
 
 
+_SHAPES = [(64, 64), (200, 50), (256, 256), (512, 512), (640, 160), (1024, 1024), (1025, 1025), (1472, 1472),
+           (2048, 512), (2560, 2560), (4096, 1024), (5000, 5000), (8191, 8191)]
+
+
 # 8: no block; 9: the first block at its smallest; 12 and 13: whole and uneven blocks; 52: more reads than a launch
-@pytest.mark.parametrize("reads", [8, 9, 12, 13, 21, 52])
-@pytest.mark.parametrize("width,rank", [(64, 64), (200, 50), (256, 256), (512, 512), (640, 160), (1024, 1024),
-                                        (1025, 1025), (1472, 1472), (2048, 512), (2560, 2560), (4096, 1024), (5000, 5000),
-                                        (8191, 8191)])
+# (a narrow, a wide and an unaligned row)
+@pytest.mark.parametrize("width,rank,reads", [(w, r, n) for w, r in _SHAPES for n in (8, 9, 12, 13, 21)] +
+                         [(w, w, 52) for w in (64, 1024, 1025)])
 def test_blocks_of_slots_match_accumulated_gradients(width, rank, reads):
-    if reads > 21 and width not in (64, 1024, 1025):
-        pytest.skip("one wide case of many reads is enough")
     dtype = torch.bfloat16 if reads % 2 else torch.float32
     print(f"bank blocks D={width} R={rank} reads={reads} {dtype}", flush=True)
     sources, queries, grads = _case(width, rank, reads, 9 if width > 1024 else 37, dtype)
