@@ -43,9 +43,10 @@ ARCH = "gfx950"
 GEOMETRIES = ((16, 1), (32, 1), (32, 2), (32, 3), (32, 4), (64, 3), (64, 4), (64, 5), (64, 6), (64, 8), (256, 3), (256, 4))
 # geometries built as two units (ATTNRES_UNIT_PART 1: forwards and gather;
 # 2: backwards, and for (64, 8) the masked forwards), with extra flags for
-# part 2: the (64, 8) backwards (streaming, key-resident, recompute) are
-# 0.4-1.2% faster with the iterative-minreg scheduler and its masked forwards
-# 1-2%, its unmasked forwards are not (MI355X, backward us, default -> minreg:
+# part 2: the (64, 8) backwards (streaming, key-resident, unmasked recompute;
+# the masked recompute is the (64, 6) unit's) are 0.4-1.2% faster with the
+# iterative-minreg scheduler and its masked forwards 1-2%, its unmasked
+# forwards are not (MI355X, backward us, default -> minreg:
 # S = 16, D = 4096, R = 1024: 777.7 / 786.7 -> 772.7 / 777.5; S = 25, R = D:
 # 1287.9 -> 1282.8; S = 25, R = 1024: 1277.8 -> 1267.3; forwards: see
 # launch_fwd)

@@ -2667,6 +2667,30 @@ int64_t launch_bwd_recompute(const BwdArgs<Rows, Grads>& a, hipStream_t stream) 
   return launch_bwd_recompute_rows<G, CH, kRecomputeMaxSources, NOMASK, VEC>(a, stream);
 }
 
+// Rows of 2048 < D <= 4096 recompute with 256 lanes of 2 chunks (recompute_lanes),
+// whichever of 64 lanes x 5, 6 or 8 chunks their other kernels take.  The masked
+// instances are compiled once, with the default scheduler: a copy in each of
+// those units, the (64, 8) one under iterative-minreg, left the choice to the
+// linker.  Measured on MI355X (backward, us, iterative-minreg -> default, N =
+// 16384): D = 4096, R = 1024: S = 1 95.1 -> 85.5, S = 2 139.2 -> 131.0, S = 3
+// 174.9 -> 183.5, S = 4 259.3 -> 231.9, S = 6 335.8 -> 340.9; D = R = 3072: S = 2
+// 112.1 -> 104.2, S = 3 133.3 -> 138.7, S = 4 223.6 -> 181.5, S = 6 269.8 ->
+// 249.7; at N = 4096 only S = 3, D = 4096 is slower (52.7 -> 55.3).
+#define ATTNRES_RECOMPUTE_256_2(KIND)                                                        \
+  KIND template int64_t launch_bwd_recompute<256, 2, false, true, PackedRows, PackedGrads>(  \
+      const BwdArgs<PackedRows, PackedGrads>&, hipStream_t);                                 \
+  KIND template int64_t launch_bwd_recompute<256, 2, false, false, PackedRows, PackedGrads>( \
+      const BwdArgs<PackedRows, PackedGrads>&, hipStream_t);                                 \
+  KIND template int64_t launch_bwd_recompute<256, 2, false, true, ListRows, ListGrads>(      \
+      const BwdArgs<ListRows, ListGrads>&, hipStream_t);                                     \
+  KIND template int64_t launch_bwd_recompute<256, 2, false, false, ListRows, ListGrads>(     \
+      const BwdArgs<ListRows, ListGrads>&, hipStream_t);
+#if defined(ATTNRES_LANES) && ATTNRES_LANES == 64 && (ATTNRES_CHUNKS == 5 || ATTNRES_CHUNKS == 8)
+ATTNRES_RECOMPUTE_256_2(extern)
+#elif defined(ATTNRES_LANES) && ATTNRES_LANES == 64 && ATTNRES_CHUNKS == 6
+ATTNRES_RECOMPUTE_256_2()
+#endif
+
 // The key-resident backward for reads of kRecomputeMaxSources < S <=
 // kKeyResMaxSources whose key is KC = keyres_key_chunks(D, R) whole chunk
 // columns (the host checks this before choosing the recompute path).
@@ -2751,10 +2775,11 @@ int64_t launch_bwd_keyres(const BwdArgs<Rows, Grads>& a, bool vec, hipStream_t s
   return 0;  // not reached: the host accepts such reads only where keyres_key_chunks applies
 }
 
-// The recompute kernel keeps S rows per lane: for the (64, 8) geometry
-// (2048 < D <= 4096) it runs with a whole workgroup per token instead, two
-// chunks per lane (same lane positions covered, so the same NOMASK rule);
-// its grid counts those groups (one token per workgroup).
+// The recompute kernel keeps S rows per lane: for 64 lanes of 5, 6 or 8 chunks
+// (2048 < D <= 4096) it runs with a whole workgroup per token instead, two chunks
+// per lane; its grid counts those groups (one token per workgroup).  At 8 chunks
+// the lane positions are the same and so is the NOMASK rule; at 5 and 6 the wider
+// group covers more than the row and is always masked.
 template <int G, int CH, class Rows, class Grads>
 int64_t launch_bwd_recompute_geometry(const BwdArgs<Rows, Grads>& a, bool nomask, bool vec, hipStream_t stream) {
   if (a.n_sources > kRecomputeMaxSources) return launch_bwd_keyres<G, CH>(a, vec, stream);
@@ -2808,6 +2833,29 @@ void launch_gather(const GatherArgs& a, hipStream_t stream) {
     launch_gather_ring<G, CH, VEC, BF16OUT, 2, 1>(a, stream);
   }
 }
+
+// Several row geometries share a gather (launch_gather_geometry): it is compiled
+// once, with the widest of them.
+#define ATTNRES_GATHERS(KIND, G, CH)                                                     \
+  KIND template void launch_gather<G, CH, true, true>(const GatherArgs&, hipStream_t);   \
+  KIND template void launch_gather<G, CH, true, false>(const GatherArgs&, hipStream_t);  \
+  KIND template void launch_gather<G, CH, false, true>(const GatherArgs&, hipStream_t);  \
+  KIND template void launch_gather<G, CH, false, false>(const GatherArgs&, hipStream_t);
+#if defined(ATTNRES_LANES)
+#if ATTNRES_LANES == 32 && ATTNRES_CHUNKS == 3
+ATTNRES_GATHERS(extern, 128, 1)
+#elif ATTNRES_LANES == 32 && ATTNRES_CHUNKS == 4
+ATTNRES_GATHERS(, 128, 1)
+#elif ATTNRES_LANES == 64 && ATTNRES_CHUNKS == 3
+ATTNRES_GATHERS(extern, 256, 1)
+#elif ATTNRES_LANES == 64 && ATTNRES_CHUNKS == 4
+ATTNRES_GATHERS(, 256, 1)
+#elif ATTNRES_LANES == 64 && (ATTNRES_CHUNKS == 5 || ATTNRES_CHUNKS == 6)
+ATTNRES_GATHERS(extern, 256, 2)
+#elif ATTNRES_LANES == 64 && ATTNRES_CHUNKS == 8 && ATTNRES_UNIT_PART == 1
+ATTNRES_GATHERS(, 256, 2)
+#endif
+#endif
 
 // The gather has no group sums, so a row is spread over up to a whole
 // workgroup with as few chunks per lane as the width allows (fewer registers:

@@ -114,3 +114,21 @@ def test_scheduler_units_hold_the_only_definitions():
         plain_lines, scheduled_lines = symbol_lines(plain, needle), symbol_lines(scheduled, needle)
         assert plain_lines and all(line.split()[0] == "U" for line in plain_lines), plain
         assert scheduled_lines and all(line.split()[1] in ("W", "T") for line in scheduled_lines), scheduled
+
+
+def test_no_kernel_is_compiled_in_two_units():
+    """Two units that instantiate one kernel may build it with different
+    scheduler options, and the linker keeps either copy without a word."""
+    nm = shutil.which("nm")
+    objects = [build_native.BUILD_DIR / name for name in _units()]
+    if nm is None or not all(obj.exists() for obj in objects):
+        pytest.skip("objects not built or nm missing")
+    units = {}
+    for obj in objects:
+        out = subprocess.run([nm, "-C", "--defined-only", str(obj)], capture_output=True, text=True, check=True).stdout
+        # a kernel's handle; its host launch stub carries the same name
+        for name in set(re.findall(r"(attnres_\w+_kernel<.*)", out)):
+            if "device_stub" not in name:
+                units.setdefault(name, set()).add(obj.name)
+    assert units
+    assert not {name: where for name, where in units.items() if len(where) > 1}
