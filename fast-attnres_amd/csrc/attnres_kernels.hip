@@ -2560,12 +2560,32 @@ void launch_fwd_geometry(const FwdArgs<Rows>& a, bool nomask, bool vec, hipStrea
 // Measured on MI355X (backward op, us): one resident grid -> two: c2 629 ->
 // 617-624, c3 833 -> 827-829; two -> four on another box: c2 618 -> 627, c3
 // 824 -> 826, c4 481 -> 486 (four: 2048 partial rows, a reduction of 11 us).
+// The geometries of 3 chunks take two workgroups per CU where that gives every
+// group at least two tokens: their fewer registers would let up to six stay, and
+// the partial rows of so many cost more than the tail they save.  Groups that are
+// not a whole workgroup also need full rounds (a fifth idle at most).  Measured on
+// MI355X (backward us, two resident grids -> two per CU): D = R = 6144: S = 8, N =
+// 1024: 70.5 -> 55.1, N = 16384: 723 -> 672; S = 48, N = 1024: 266 -> 223; D = 5120,
+// R = 1280: S = 8, N = 1024: 52.4 -> 45.2; S = 25, N = 8192: 811 -> 803; D = R = 1536:
+// S = 25, N = 4096: 131.8 -> 123.3, N = 16384: 501 -> 482; D = R = 768, N = 8192: S = 8
+// 49.4 -> 44.5, S = 48 234.9 -> 218.6; but S = 48, N = 6000 (1.5 rounds): 164 -> 195,
+// S = 25, N = 8800 (2.15): 131 -> 143, and at 256 lanes N = 1100 (2.15), D = R = 6144:
+// S = 7 69.3 -> 59.7, S = 25 155.2 -> 155.9.
 constexpr int64_t kBwdGridPerResident = 2;
+template <int G, int CH>
+int64_t bwd_grid(int64_t n_tokens, int64_t resident) {
+  if constexpr (CH == 3) {
+    const int64_t two_per_cu = 2 * device_cus(), at_once = kBlock / G * two_per_cu;  // tokens per round
+    const auto rounds = [&] { return (n_tokens + at_once - 1) / at_once; };
+    if (at_once > 0 && n_tokens >= 2 * at_once && (G == kBlock || 5 * n_tokens >= 4 * rounds() * at_once)) return two_per_cu;
+  }
+  return kBwdGridPerResident * resident;
+}
 
 template <int G, int CH, int NB, bool NOMASK, bool VEC, bool ACC, class Rows, class Grads>
 int64_t launch_bwd_ring(const BwdArgs<Rows, Grads>& a, hipStream_t stream) {
   const int64_t resident = resident_blocks<&attnres_bwd_kernel<G, CH, NB, NOMASK, VEC, ACC, Rows, Grads>>();
-  const int64_t blocks = grid_blocks(a.n_tokens, G, kBwdGridPerResident * resident, a.max_grid);
+  const int64_t blocks = grid_blocks(a.n_tokens, G, bwd_grid<G, CH>(a.n_tokens, resident), a.max_grid);
   hipLaunchKernelGGL((attnres_bwd_kernel<G, CH, NB, NOMASK, VEC, ACC, Rows, Grads>),
                      dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a);
   return blocks;
@@ -2649,10 +2669,30 @@ int64_t launch_bwd_geometry(const BwdArgs<Rows, Grads>& a, bool nomask, bool vec
              : launch_bwd_variant<G, CH, false>(a, nomask, vec, stream);
 }
 
+// The recompute backward's grid is one resident one.  The aligned geometries of 3
+// chunks have the registers for more workgroups, whose dq partial rows and query
+// copies then cost more than the tokens they share: a read that gives each group
+// of one workgroup per CU two to four tokens, and the workgroup at most 32 rows,
+// takes that grid, and one of more tokens at 256 lanes two workgroups per CU.
+// Measured on MI355X (backward us, resident grid -> this): D = R = 6144: S = 1, N =
+// 512: 23.5 -> 17.3, N = 1024: 33.5 -> 22.3, N = 2048: 39.4 -> 34.0, N = 16384: 133.8 ->
+// 129.3; S = 6, N = 1024: 46.7 -> 42.4; D = R = 1536: S = 1, N = 2048: 11.3 -> 9.6, N =
+// 4096: 17.5 -> 14.7, S = 2, N = 4096: 19.8 -> 17.3; but one workgroup per CU at S = 6,
+// N = 4096: 35.9 -> 37.4, S = 1, N = 16384: 37.1 -> 41.4 (two per CU: 37.5).
+template <int G, int CH, bool VEC>
+int64_t recompute_grid(int64_t n_tokens, int n_sources, int64_t resident) {
+  if constexpr (CH == 3 && G >= 64 && VEC) {
+    const int64_t cus = device_cus(), per_cu = kBlock / G * cus;  // tokens that one workgroup per CU takes at once
+    if (n_tokens >= 2 * per_cu && n_tokens <= 4 * per_cu && n_tokens * n_sources <= 32 * cus && cus < resident) return cus;
+    if (G == kBlock && n_tokens > 2 * cus && 2 * cus < resident) return 2 * cus;
+  }
+  return resident;
+}
+
 template <int G, int CH, int SM, bool NOMASK, bool VEC, class Rows, class Grads>
 int64_t launch_bwd_recompute_rows(const BwdArgs<Rows, Grads>& a, hipStream_t stream) {
   const int64_t resident = resident_blocks<&attnres_bwd_recompute_kernel<G, CH, SM, NOMASK, VEC, Rows, Grads>>();
-  const int64_t blocks = grid_blocks(a.n_tokens, G, resident, a.max_grid);
+  const int64_t blocks = grid_blocks(a.n_tokens, G, recompute_grid<G, CH, VEC>(a.n_tokens, a.n_sources, resident), a.max_grid);
   hipLaunchKernelGGL((attnres_bwd_recompute_kernel<G, CH, SM, NOMASK, VEC, Rows, Grads>),
                      dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, stream, a);
   return blocks;
