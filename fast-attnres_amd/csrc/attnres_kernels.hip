@@ -2395,16 +2395,26 @@ void launch_fwd_block(const FwdArgs<Rows>& a, hipStream_t stream) {
 // D = 2048: 56.9 -> 11.8, S = 9, D = 8192: 21.7 -> 18.0, S = 25, D = 256: 19.2
 // -> 7.8; 512 tokens: S = 25, D = 1024: 19.5 -> 13.7, S = 48, D = 2048: 35.4 ->
 // 32.2, S = 3: 6.6 -> 6.5; but S = 9, D = 4096: 16.3 -> 19.8, D = 8192: 23.5 ->
-// 33.5, and 1024 tokens, S = 25, D = 1024: 20.2 -> 35.  Reads of one source
-// have no second row to wait for and keep the streaming kernel.
-inline bool few_tokens(int64_t n_tokens, int width) {
+// 33.5, and 1024 tokens, S = 25, D = 1024: 20.2 -> 35.
+// * Rows of up to 256 elements (16 lanes, or 32 lanes of one chunk) only from 4
+//   sources: fewer are in flight at once anyway (512 tokens, S = 2: D = 64: 2.8 ->
+//   3.3, D = 200: 2.9 -> 3.4; S = 3: 3.1 -> 3.3).
+// * 64 lanes x 3 (1024 < D <= 1536) past one per CU only from 9 sources: their 768
+//   threads leave no room for a second workgroup on a CU (512 tokens, D = 1536:
+//   S = 2 4.5 -> 6.5, S = 4 5.5 -> 6.7, S = 8 6.9 -> 7.4; S = 12 8.3 -> 8.0, S = 25, D =
+//   1280 13.7 -> 12.1).
+// * Reads of one source are left to the streaming kernel (not compared).
+template <int G, int CH>
+bool few_tokens(int64_t n_tokens, int n_sources, int width) {
+  if (n_sources < (G * CH <= 32 ? 4 : 2)) return false;
   const int64_t cus = device_cus();
-  return n_tokens <= (width <= 2048 ? 2 * cus : cus);
+  const bool two = width <= 2048 && (G != 64 || CH != 3 || n_sources >= 9);
+  return n_tokens <= (two ? 2 * cus : cus);
 }
 
 template <int G, int CH, bool VEC, class Rows>
 bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
-  if (a.n_sources < 2 || !few_tokens(a.n_tokens, a.width)) return false;
+  if (!few_tokens<G, CH>(a.n_tokens, a.n_sources, a.width)) return false;
   constexpr int kColumnThreads = G * CH * kVec / few_columns(G, CH);
   int threads = (a.n_sources * G + 63) / 64 * 64;
   if (threads < kColumnThreads) threads = kColumnThreads;

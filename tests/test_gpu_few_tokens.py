@@ -70,3 +70,20 @@ def test_few_tokens_with_special_values(width):
         for n, one in enumerate(few):
             torch.testing.assert_close(one[2], whole[2][n:n + 1], rtol=0, atol=0, equal_nan=True)
             torch.testing.assert_close(one[0], whole[0][n:n + 1], rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("sources,width", [(3, 256), (4, 256), (2, 64), (8, 1536), (9, 1536), (8, 1025), (9, 1025), (2, 2048)])
+def test_both_sides_of_one_and_two_tokens_per_cu(sources, width):
+    """Whether a few tokens' read runs one workgroup per token also depends on
+    its width and sources: around 256 and 512 tokens (a CU each, two) the bits
+    are those of the same tokens of a large read."""
+    torch.manual_seed(sources + width)
+    values = torch.randn(sources, 3000, width, device="cuda", dtype=torch.bfloat16)
+    query = (torch.randn(width, device="cuda") * 3 / math.sqrt(width)).to(torch.bfloat16)
+    whole = _ops.packed_forward_impl(values, query, 2**-23, 1.0, True)
+    for count in (256, 257, 512, 513):
+        few = _ops.packed_forward_impl(values[:, :count], query, 2**-23, 1.0, True)
+        torch.cuda.synchronize()
+        for a, b in zip(few[:4], whole):
+            assert torch.equal(a, b[:count])
+        assert torch.equal(few[4], whole[4][:, :count])
