@@ -2452,7 +2452,10 @@ bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
 //   - 32 x 2 and 32 x 3: 2 x 2 (D = 512, S = 25: ring 87.7 -> 76.0; D = 640,
 //     N = 8192: ring 58.8, 2 x 1 53.0, 2 x 2 48.3);
 //   - 32 x 4, from 9 sources: 2 x 2 on whole rows (D = 1024, S = 13: ring 87.4
-//     -> 78.8, S = 25: 148.7 -> 140.0; S = 5: 39.0 -> 39.8), 2 x 1 on shorter
+//     -> 78.8, S = 25: 148.7 -> 140.0; S = 5: 39.0 -> 39.8), but 1 x 4 with key
+//     masks, aligned and up to 16 sources (R = 256, refinement saved: S = 10: ring 66.6, 2 x 2
+//     70.3, 1 x 4 63.8; S = 16: 99.7 / 97.8 / 97.3; S = 25, N = 8192: 73.3 / 71.7 /
+//     72.5; rows 2 bytes off, S = 9, no refinement: - / 66.3 / 69.0), 2 x 1 on shorter
 //     ones (D = 896, S = 9: 50.9-54.7 against 58.0-60.8 for 2 x 2);
 //   - 64 x 3: 2 x 1 (D = 1280, N = 8192, S = 25: ring 99.1 -> 94.5);
 //   - 64 x 4: short rows 2 x 1 (D = 1792, one token -> two: 81 -> 78 at S = 13);
@@ -2461,11 +2464,17 @@ bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
 //     N = 32768: ring 252.7 -> 234.6), 1 x 4 for 13 to 23 (S = 20: 234.5 ->
 //     228.3), 4 x 1 from 24 (S = 25: 1 x 4 284.5, 4 x 1 277.8; S = 49,
 //     N = 8192, cold: 298 -> 260);
-//   - 64 x 5, 64 x 6 and 256 x 3, from 9 sources: 4 x 1 (D = 2560, S = 25: ring
-//     183.9, 2 x 1 177.4, 4 x 1 170.9; D = 3072: 215.1 / 212.7 / 209.7;
-//     D = 5120, N = 4096, S = 13: 112.3 / 106.5 / 100.9), but 256 x 3 only past
-//     12 wavefronts per SIMD (D = 5120, N = 1536, S = 25: 2 x 1 75.8, 4 x 1 85.9;
-//     N = 3072: 138.4 / 147.4);
+//   - 64 x 5 and 64 x 6, from 9 sources: 4 x 1 (D = 2560, S = 25: ring 183.9,
+//     2 x 1 177.4, 4 x 1 170.9; D = 3072: 215.1 / 212.7 / 209.7);
+//   - 256 x 3: 2 x 1 for 5 to 7 sources (N = 16384, R = D / 4 at 5120: S = 6: D =
+//     5120: ring 221, 2 x 1 192, 4 x 1 192; D = 6144: 264 / 231 / 232; S = 5, N = 4096:
+//     56.1 / 53.9 / 54.0), 4 x 1 from 8 (S = 8: D = 5120: 303 / 270 / 272, D = 6144:
+//     365 / 327 / 316; D = 5120, N = 4096, S = 13: 112.3 / 106.5 / 100.9), but 4 x 1
+//     only past 12 wavefronts per SIMD (D = 5120, N = 1536, S = 25: 2 x 1 75.8, 4 x 1
+//     85.9; N = 3072: 138.4 / 147.4), 2 x 2 up to and with four (N = 1024: S = 12:
+//     D = 5120: 2 x 1 27.7, 2 x 2 25.1, D = 6144: 33.7 / 30.1; S = 25: 49.8 / 46.0, 58.7 /
+//     56.2), and up to 8 sources the ring up to there (N = 1100: S = 7: D = 5120: 18.2,
+//     2 x 1 19.9; D = 6144: 21.9 / 24.7; N = 2048, D = 6144: S = 6 30.3 / 31.4);
 //   - 64 x 8, past 12 sources: 2 x 1 (D = 4096, S = 25, N = 16384: ring 601 ->
 //     588; S = 5 with two tokens instead of the persistent ring: 135 -> 153);
 //   - 256 x 4: 2 x 1 (D = 8192, N = 8192, S = 48: ring 1160.8 -> 1134.0).
@@ -2479,19 +2488,22 @@ struct FwdBlockShape {
   int rows;    // of each in flight
 };
 
-inline FwdBlockShape fwd_block_shape(int G, int CH, bool whole, bool nomask, int S) {
+inline FwdBlockShape fwd_block_shape(int G, int CH, bool whole, bool nomask, bool vec, int S) {
   if (S < kFwdBlockMinSources || G == 16) return {0, 0};
   if (G == 32) {
     if (CH == 1) return {1, 4};
     if (CH < 4) return {2, 2};
-    return S < 9 ? FwdBlockShape{0, 0} : whole ? FwdBlockShape{2, 2} : FwdBlockShape{2, 1};
+    if (S < 9) return {0, 0};
+    if (!whole) return {2, 1};
+    return !nomask && vec && S <= 16 ? FwdBlockShape{1, 4} : FwdBlockShape{2, 2};
   }
   if (CH == 8) return S > kPersistentFwdMaxSources ? FwdBlockShape{2, 1} : FwdBlockShape{0, 0};
   if (CH == 4 && G == 64 && whole) {
     if (!nomask) return {1, 4};
     return S <= 12 ? FwdBlockShape{2, 2} : S < 24 ? FwdBlockShape{1, 4} : FwdBlockShape{4, 1};
   }
-  if (CH > 4 || (G == kBlock && CH == 3)) return S < 9 ? FwdBlockShape{0, 0} : FwdBlockShape{4, 1};
+  if (G == kBlock && CH == 3) return S < 8 ? FwdBlockShape{2, 1} : FwdBlockShape{4, 1};
+  if (CH > 4) return S < 9 ? FwdBlockShape{0, 0} : FwdBlockShape{4, 1};
   return {2, 1};
 }
 
@@ -2502,18 +2514,20 @@ void launch_fwd(const FwdArgs<Rows>& a, hipStream_t stream) {
     const int64_t cus = device_cus();
     const bool whole = a.width == G * CH * kVec;
     const auto below = [&](int64_t waves_per_cu) { return a.n_tokens * G < waves_per_cu * 64 * cus; };
-    FwdBlockShape shape = fwd_block_shape(G, CH, whole, NOMASK, a.n_sources);
+    FwdBlockShape shape = fwd_block_shape(G, CH, whole, NOMASK, VEC, a.n_sources);
     if (G <= 64 && a.n_sources > 1 && few_waves(a.n_tokens, G)) {
       shape = {1, 4};
-    } else if (CH > 1 && CH < 8 && a.n_sources >= kFwdBlockMinSources && below(whole ? 16 : 8)) {
+    } else if (CH > 1 && CH < 8 && a.n_sources >= kFwdBlockMinSources &&
+               below(G == kBlock && CH == 3 && a.n_sources >= 9 ? 17 : whole ? 16 : 8)) {
       shape = {2, 2};
-    } else if (G == kBlock && CH == 3 && shape.tokens == 4 && below(49)) {
-      shape = {2, 1};
+    } else if (G == kBlock && CH == 3 && below(49)) {
+      shape = a.n_sources >= 9 ? FwdBlockShape{2, 1} : FwdBlockShape{0, 0};
     }
     // the shapes each geometry can get; a shape outside them does not compile in
     constexpr bool kOne = G <= 64;
     constexpr bool kTwoTwo = CH > 1 && CH < 8;
-    constexpr bool kTwoOne = (G == 32 && CH == 4) || (G == 64 && (CH == 3 || CH == 4 || CH == 8)) || G == kBlock;
+    // (unmasked rows of 32 or 64 lanes x 4 are whole)
+    constexpr bool kTwoOne = (CH == 4 && G < kBlock && !NOMASK) || (G == 64 && (CH == 3 || CH == 8)) || G == kBlock;
     constexpr bool kFour = (G == 64 && CH == 4 && NOMASK) || (G == 64 && (CH == 5 || CH == 6)) || (G == kBlock && CH == 3);
     if constexpr (kOne) {
       if (shape.tokens == 1) return launch_fwd_block<G, CH, 1, 4, NOMASK, VEC>(a, stream);
