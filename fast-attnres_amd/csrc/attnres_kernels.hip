@@ -2329,9 +2329,9 @@ inline int64_t device_cus() {
 // are 2-3% slower with them (S=25, N=16384, D=R=4096: 1273 -> 1316; with the
 // iterative-minreg scheduler of the (64, 8) backward unit too: S=25 1295.5 ->
 // 1329.5, S=13 715.1 -> 727.6, S=48 2487.9 -> 2514.9).
-// One row per group where rows leave chunks idle or are not aligned, whatever
-// the lanes: more wavefronts then hide more than a second row does.  Two rows ->
-// one: S = 17, N = 8192, D = 5120, R = 1280 (now 256 x 3): 664 -> 550; D = 7168,
+// Past that, one row per group where rows leave chunks idle or are not aligned,
+// whatever the lanes: more wavefronts then hide more than a second row does.  Two
+// rows -> one: S = 17, N = 8192, D = 5120, R = 1280 (now 256 x 3): 664 -> 550; D = 7168,
 // R = 1792: 808 -> 712; S = 9, N = 2048, D = 1800: 47.7 -> 40.5; D = 1537: 46.1 ->
 // 37.1.  Rows of 3 chunks per lane are level (D = 1536, N = 8192, S = 9: 100.7 /
 // 100.5) and take two rows only on small grids.
@@ -2396,17 +2396,18 @@ void launch_fwd_block(const FwdArgs<Rows>& a, hipStream_t stream) {
 // -> 7.8; 512 tokens: S = 25, D = 1024: 19.5 -> 13.7, S = 48, D = 2048: 35.4 ->
 // 32.2, S = 3: 6.6 -> 6.5; but S = 9, D = 4096: 16.3 -> 19.8, D = 8192: 23.5 ->
 // 33.5, and 1024 tokens, S = 25, D = 1024: 20.2 -> 35.
-// * Rows of up to 256 elements (16 lanes, or 32 lanes of one chunk) only from 4
-//   sources: fewer are in flight at once anyway (512 tokens, S = 2: D = 64: 2.8 ->
-//   3.3, D = 200: 2.9 -> 3.4; S = 3: 3.1 -> 3.3).
+// * Aligned rows of up to 256 elements (16 lanes, or 32 lanes of one chunk) only
+//   from 4 sources: fewer are in flight at once anyway (512 tokens, S = 2: D = 64:
+//   2.8 -> 3.3, D = 200: 2.9 -> 3.4; S = 3: 3.1 -> 3.3; but unaligned, 64 tokens, S = 3,
+//   D = 255: 3.7 -> 3.3).
 // * 64 lanes x 3 (1024 < D <= 1536) past one per CU only from 9 sources: their 768
 //   threads leave no room for a second workgroup on a CU (512 tokens, D = 1536:
 //   S = 2 4.5 -> 6.5, S = 4 5.5 -> 6.7, S = 8 6.9 -> 7.4; S = 12 8.3 -> 8.0, S = 25, D =
 //   1280 13.7 -> 12.1).
 // * Reads of one source are left to the streaming kernel (not compared).
-template <int G, int CH>
+template <int G, int CH, bool VEC>
 bool few_tokens(int64_t n_tokens, int n_sources, int width) {
-  if (n_sources < (G * CH <= 32 ? 4 : 2)) return false;
+  if (n_sources < (G * CH <= 32 && VEC ? 4 : 2)) return false;
   const int64_t cus = device_cus();
   const bool two = width <= 2048 && (G != 64 || CH != 3 || n_sources >= 9);
   return n_tokens <= (two ? 2 * cus : cus);
@@ -2414,7 +2415,7 @@ bool few_tokens(int64_t n_tokens, int n_sources, int width) {
 
 template <int G, int CH, bool VEC, class Rows>
 bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
-  if (!few_tokens<G, CH>(a.n_tokens, a.n_sources, a.width)) return false;
+  if (!few_tokens<G, CH, VEC>(a.n_tokens, a.n_sources, a.width)) return false;
   constexpr int kColumnThreads = G * CH * kVec / few_columns(G, CH);
   int threads = (a.n_sources * G + 63) / 64 * 64;
   if (threads < kColumnThreads) threads = kColumnThreads;
@@ -2439,25 +2440,30 @@ bool launch_fwd_few(const FwdArgs<Rows>& a, hipStream_t stream) {
 //   N = 1024: 59.4 (4 x 1) -> 20.9; D = 2560, N = 768: 28.5 -> 21.2; D = 768,
 //   N = 2048: 35.2 (2 x 1) -> 17.1.
 // * Below four per SIMD (two where rows leave chunks idle): two tokens, two rows
-//   of each: the blocks still fill the chip and keep adjacent rows in flight.  S = 25, 1 x 4 / ring / larger
-//   block -> 2 x 2: D = 2048, N = 2048: 39.4 / 39.9 / 63.7 -> 37.1, N = 3072:
-//   - / 59.5 / 68.4 -> 59.2, but N = 4096 eager: - / - / 70.1 -> 71.2; D = 1536, N = 2048: 30.4 / 31.3 / 53.0 -> 28.7;
-//   D = 1024, N = 4096: 39.8 / 40.6 / 52.5 -> 37.6; D = 8192, N = 1024: 76.0 /
-//   77.9 / 77.0 -> 75.5.  (64, 8) groups keep the choice below (N = 2048,
-//   S = 25: 80.6 against 76.0).
+//   of each: the blocks still fill the chip and keep adjacent rows in flight.
+//   S = 25, 1 x 4 / ring / larger block -> 2 x 2: D = 2048, N = 2048: 39.4 / 39.9 /
+//   63.7 -> 37.1, N = 3072: - / 59.5 / 68.4 -> 59.2, but N = 4096 eager: - / - /
+//   70.1 -> 71.2; D = 1536, N = 2048: 30.4 / 31.3 / 53.0 -> 28.7; D = 1024, N =
+//   4096: 39.8 / 40.6 / 52.5 -> 37.6; D = 8192, N = 1024: 76.0 / 77.9 / 77.0 ->
+//   75.5.  (64, 8) groups keep the choice below (N = 2048, S = 25: 80.6 against
+//   76.0).
 // * Beyond, by geometry (fwd_block_shape): what keeps most rows of adjacent
-//   tokens in flight without spilling, N = 16384 for D <= 2048, else 8192:
+//   tokens in flight without scratch memory (64 x 5 and 64 x 6 with four tokens keep
+//   63 to 189 values in AGPRs), N = 16384 for D <= 2048, else 8192:
 //   - 32 lanes x 1: 1 x 4 (D = 256, S = 25: ring 52.0, 2 x 2 48.9, 1 x 4 47.6;
 //     N = 8192: 28.6 / 28.6 / 26.2);
 //   - 32 x 2 and 32 x 3: 2 x 2 (D = 512, S = 25: ring 87.7 -> 76.0; D = 640,
-//     N = 8192: ring 58.8, 2 x 1 53.0, 2 x 2 48.3);
+//     N = 8192: ring 58.8, 2 x 1 53.0, 2 x 2 48.3; only masked whole rows of 768 and
+//     many sources are better with 2 x 1: R = 192, S = 16 66.7 / 67.3, S = 25 102.2 /
+//     106.8, S = 48 196.2 / 203.0, but N = 4096, S = 25 34.0 / 26.2);
 //   - 32 x 4, from 9 sources: 2 x 2 on whole rows (D = 1024, S = 13: ring 87.4
 //     -> 78.8, S = 25: 148.7 -> 140.0; S = 5: 39.0 -> 39.8), but 1 x 4 with key
-//     masks, aligned and up to 16 sources (R = 256, refinement saved: S = 10: ring 66.6, 2 x 2
-//     70.3, 1 x 4 63.8; S = 16: 99.7 / 97.8 / 97.3; S = 25, N = 8192: 73.3 / 71.7 /
-//     72.5; rows 2 bytes off, S = 9, no refinement: - / 66.3 / 69.0), 2 x 1 on shorter
-//     ones (D = 896, S = 9: 50.9-54.7 against 58.0-60.8 for 2 x 2);
-//   - 64 x 3: 2 x 1 (D = 1280, N = 8192, S = 25: ring 99.1 -> 94.5);
+//     masks, aligned and up to 16 sources (R = 256, refinement saved: S = 10: ring
+//     66.6, 2 x 2 70.3, 1 x 4 63.8; S = 16: 99.7 / 97.8 / 97.3; S = 25, N = 8192: 73.3 /
+//     71.7 / 72.5; rows 2 bytes off, S = 9, no refinement: - / 66.3 / 69.0), 2 x 1 on
+//     shorter ones (D = 896, S = 9: 50.9-54.7 against 58.0-60.8 for 2 x 2);
+//   - 64 x 3: 2 x 1 (D = 1280, N = 8192, S = 25: ring 99.1 -> 94.5; S = 48: 4 x 1 170.9,
+//     2 x 1 179.0, N = 16384 345 / 354, but N = 4096 87.4 / 84.0);
 //   - 64 x 4: short rows 2 x 1 (D = 1792, one token -> two: 81 -> 78 at S = 13);
 //     whole rows with key masks 1 x 4 (R = 512, S = 25: ring 297 -> 282; S = 16:
 //     190 -> 177); whole rows without: 2 x 2 for 5 to 12 sources (S = 9,
@@ -2739,7 +2745,8 @@ int64_t launch_bwd_recompute(const BwdArgs<Rows, Grads>& a, hipStream_t stream) 
 // 16384): D = 4096, R = 1024: S = 1 95.1 -> 85.5, S = 2 139.2 -> 131.0, S = 3
 // 174.9 -> 183.5, S = 4 259.3 -> 231.9, S = 6 335.8 -> 340.9; D = R = 3072: S = 2
 // 112.1 -> 104.2, S = 3 133.3 -> 138.7, S = 4 223.6 -> 181.5, S = 6 269.8 ->
-// 249.7; at N = 4096 only S = 3, D = 4096 is slower (52.7 -> 55.3).
+// 249.7; at D = 4096, R = 1024 also N = 4096, S = 3 52.7 -> 55.3, N = 2048, S = 6 47.8 ->
+// 52.6.
 #define ATTNRES_RECOMPUTE_256_2(KIND)                                                        \
   KIND template int64_t launch_bwd_recompute<256, 2, false, true, PackedRows, PackedGrads>(  \
       const BwdArgs<PackedRows, PackedGrads>&, hipStream_t);                                 \
