@@ -224,14 +224,18 @@ class SourceBank:
     no dv rows, only its dq and the per-token coefficients of its dv
     (``attnres_hip_{packed,sources}_backward_coef``), and keeps its BF16 dO.
     Slot i's gradient is formed once, when the slot's push node runs its
-    backward, by ``attnres_hip_bank_gather``: one FP32 pass over the dO rows
-    of the reads that saw slot i.  The ordering uses one chain of zero-size
-    tokens: every push node takes the token of the push before it, and a
-    read takes the latest token, so a push node's backward runs after that
-    of every read made after the push (those that saw the slot among them),
-    and a read has one token input however many slots it reads.  ``gradients="accumulate"`` instead adds
-    every read's FP32 dv into one FP32 ``[capacity, ..., D]`` buffer in the
-    backward kernel (``attnres_hip_{packed,sources}_backward_accumulate_f32``:
+    backward, by ``attnres_hip_bank_gather_slots``: one FP32 pass over the dO
+    rows of the reads that saw slot i.  From nine such reads on the same pass
+    also forms the sums of the three slots before it, where the backward pass
+    computes their gradients too, and these add their later reads to them (12
+    more bytes per element of a source at the peak of the pass).  The ordering
+    uses one chain of zero-size tokens: every push node takes the token of the
+    push before it, and a read takes the latest token, so a push node's backward
+    runs after that of every read made after the push (those that saw the slot
+    among them), and a read has one token input however many slots it reads.
+    ``gradients="accumulate"`` instead adds every read's FP32 dv into one FP32
+    ``[capacity, ..., D]`` buffer in the backward kernel
+    (``attnres_hip_{packed,sources}_backward_accumulate_f32``:
     a read-modify-write of the sum per read).  Either way the sums are FP32
     without BF16 rounding of the per-read dv, and reach the source in its
     dtype.  Eager mode only; one bank per forward pass.
