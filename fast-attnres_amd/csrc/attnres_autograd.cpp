@@ -657,7 +657,9 @@ struct BankPushSum : public torch::autograd::Function<BankPushSum> {
     if (grad.defined()) grad = grad.to(dtype);
     if (grads[0].defined()) grad = grad.defined() ? grads[0] + grad : grads[0];
     // neither the partial nor the slot was used: a zero gradient, not an absent one
-    if (!grad.defined()) grad = torch::zeros(bank->values.sizes().slice(1), bank->values.options().dtype(dtype));
+    if (!grad.defined() && (ctx->needs_input_grad(0) || ctx->needs_input_grad(1))) {
+      grad = torch::zeros(bank->values.sizes().slice(1), bank->values.options().dtype(dtype));
+    }
     const bool token = ctx->saved_data["token"].toBool();
     return {Tensor(), Tensor(), grad, grad, token ? torch::empty({0}, bank->values.options().dtype(dtype)) : Tensor()};
   }
